@@ -41,7 +41,9 @@ typedef enum nq_status {
 
 typedef enum nq_dtype { NQ_F32 = 0, NQ_F16 = 1 } nq_dtype;
 
-/* Kernel selection for the W8A8 linears. AUTO: m <= 4 (m <= 8 when k >= 4096 or n >= 8192)
+/* Kernel selection for the W8A8 linears. AUTO: operands that fit neither the GEMVs nor the
+ * MFMA kernels (k % 16, alignment), from m = 9, and k % 64 past m = 128 -> the tile GEMM over
+ * any k; else m <= 4 (m <= 8 when k >= 4096 or n >= 8192)
  * -> workgroup-per-rows GEMV (v_dot4_i32_i8), larger m -> int8 MFMA GEMM; nq_linear_w8a8 runs
  * m = 1 as one GEMV launch with the act quant fused in, and with AUTO tries the one-launch
  * decode kernel (m * k <= 4096, or m <= 4 and m * k <= 8192) and the decode kernel over the act quant's codes
@@ -134,6 +136,9 @@ nq_status nq_linear_q8(const void* x, nq_dtype x_dtype, const int8_t* q, const f
  * NULL is accepted), 256-byte aligned. No counterpart in the reference, whose
  * cuda_linear_q8 (cuda_quant.cu:300-322) takes no workspace. */
 size_t nq_linear_wq_workspace_size(int64_t m, int64_t n, int64_t k);
+/* The workspace with which every kernel choice at this shape can split K as far as it
+ * gains: at least nq_linear_wq_workspace_size, which remains what the calls require. */
+size_t nq_linear_wq_workspace_preferred(int64_t m, int64_t n, int64_t k);
 nq_status nq_linear_q8_ws(const void* x, nq_dtype x_dtype, const int8_t* q, const float* w_scale,
                           const float* bias, void* y, nq_dtype y_dtype, int64_t m, int64_t n, int64_t k,
                           void* workspace, size_t workspace_bytes, void* stream);
@@ -230,6 +235,8 @@ nq_status nq_linear_q4g_ex(const void* x, nq_dtype x_dtype, const uint8_t* q, co
  * workspace: >= nq_linear_w8a8_workspace_size(m, n, k) bytes, 256-byte aligned;
  * the reference allocated xq/a_scale per call (cuda_quant.cu:253-258). */
 size_t nq_linear_w8a8_workspace_size(int64_t m, int64_t n, int64_t k);
+/* As nq_linear_wq_workspace_preferred: at least the required size. */
+size_t nq_linear_w8a8_workspace_preferred(int64_t m, int64_t n, int64_t k);
 nq_status nq_linear_w8a8(const void* x, nq_dtype x_dtype, const int8_t* wq, const float* w_scale,
                          const float* bias, void* y, nq_dtype y_dtype, int64_t m, int64_t n,
                          int64_t k, void* workspace, size_t workspace_bytes, int path,
@@ -239,6 +246,7 @@ nq_status nq_linear_w8a8(const void* x, nq_dtype x_dtype, const int8_t* wq, cons
  * nq_act_quant_i8) — the GEMM half of cuda_linear_w8a8 (cuda_quant.cu:260-283).
  * workspace: >= nq_gemm_w8a8_workspace_size(m, n, k) bytes (split-K partials). */
 size_t nq_gemm_w8a8_workspace_size(int64_t m, int64_t n, int64_t k);
+size_t nq_gemm_w8a8_workspace_preferred(int64_t m, int64_t n, int64_t k);
 nq_status nq_gemm_w8a8(const int8_t* xq, const float* a_scale, const int8_t* wq,
                        const float* w_scale, const float* bias, void* y, nq_dtype y_dtype,
                        int64_t m, int64_t n, int64_t k, void* workspace, size_t workspace_bytes,

@@ -271,7 +271,7 @@ Tensor linear_q8_path(const Tensor& x, const QTensor& w, const Tensor* bias, DTy
     require(x.size(1) == w.in, "linear_q8: x cols must match weight in-features");
     const float* b = bias_ptr(bias, w.out, "linear_q8: bias must be a device fp32 tensor");
     Tensor y({x.size(0), w.out}, out_dtype, Device::HIP);
-    const size_t need = nq_linear_wq_workspace_size(x.size(0), w.out, w.in);
+    const size_t need = nq_linear_wq_workspace_preferred(x.size(0), w.out, w.in);
     void* ws = need ? workspace(need) : nullptr;
     nq_check(nq_linear_q8_ex(x.device_ptr(), abi_dtype(x.dtype()), static_cast<const int8_t*>(w.q.device_ptr()),
                              static_cast<const float*>(w.scale.device_ptr()), b, y.device_ptr(),
@@ -289,7 +289,7 @@ Tensor linear_w8a8(const Tensor& x, const QTensor& w, const Tensor* bias, DType 
     require(x.size(1) == w.in, "linear_w8a8: x cols must match weight in-features");
     const float* b = bias_ptr(bias, w.out, "linear_w8a8: bias must be a device fp32 tensor");
     Tensor y({x.size(0), w.out}, out_dtype, Device::HIP);
-    const size_t need = nq_linear_w8a8_workspace_size(x.size(0), w.out, w.in);
+    const size_t need = nq_linear_w8a8_workspace_preferred(x.size(0), w.out, w.in);
     void* ws = need ? workspace(need) : nullptr;
     nq_check(nq_linear_w8a8(x.device_ptr(), abi_dtype(x.dtype()), static_cast<const int8_t*>(w.q.device_ptr()),
                             static_cast<const float*>(w.scale.device_ptr()), b, y.device_ptr(),
@@ -302,7 +302,7 @@ Tensor linear_q4g(const Tensor& x, const Q4GTensor& w, const Tensor* bias, DType
     require(x.size(1) == w.in, "linear_q4g: x cols must match weight in-features");
     const float* b = bias_ptr(bias, w.out, "linear_q4g: bias must be a device fp32 tensor");
     Tensor y({x.size(0), w.out}, out_dtype, Device::HIP);
-    const size_t need = nq_linear_wq_workspace_size(x.size(0), w.out, w.in);
+    const size_t need = nq_linear_wq_workspace_preferred(x.size(0), w.out, w.in);
     void* ws = need ? workspace(need) : nullptr;
     nq_check(nq_linear_q4g_ws(x.device_ptr(), abi_dtype(x.dtype()), static_cast<const uint8_t*>(w.q.device_ptr()),
                               w.scale.device_ptr(), abi_dtype(w.scale.dtype()), w.group, b, y.device_ptr(),

@@ -19,6 +19,7 @@
 
 #include "nq_device.hpp"
 #include "nq_internal.hpp"
+#include "nq_tile_gemm.hpp"
 
 namespace nq {
 bool wq_gemm_ok(bool q4, const void* x, size_t x_elem, const void* w, int64_t m, int64_t n, int64_t k,
@@ -27,6 +28,9 @@ template <bool Q4, typename XT, typename YT, typename ST>
 nq_status wq_gemm(const XT* x, const uint8_t* w, const ST* sc, const float* b, YT* y, int64_t m, int64_t n,
                   int64_t k, int64_t group, void* workspace, size_t workspace_bytes, hipStream_t s);
 size_t wq_workspace_bytes(int64_t m, int64_t n, int64_t k);
+bool wq_tile_route(bool q4, bool f32x, bool scale_f16, bool general, bool slices, int64_t m, int64_t n, int64_t k,
+                   int64_t group, bool ws);
+size_t wq_tile_ws_bytes(int64_t m, int64_t n, int64_t k);
 
 namespace {
 
@@ -2563,10 +2567,17 @@ nq_status linear_q8_impl(const void* x, nq_dtype x_dtype, const int8_t* q, const
                NQ_BAD_ALIGN, "linear_q8: misaligned pointer");
     hipStream_t s = as_stream(stream);
     const int ni = static_cast<int>(n), ki = static_cast<int>(k);
-    // Batched activations: the fp16 MFMA GEMM when the shape rule in wq_gemm_ok
-    // picks it, else GEMV slices of 8 rows.
+    const bool aligned16 = aligned(q, 16) && aligned(x, 16);
+    const bool fast = path != NQ_PATH_GENERIC && k % 16 == 0 && k > 0 && k / 16 <= kMaxGemvThreads && aligned16;
+    const bool long_k = path != NQ_PATH_GENERIC && k % 16 == 0 && k / 16 > kMaxGemvThreads && aligned16;
+    // Batched activations: the tile GEMM where wq_tile_route picks it, the MFMA GEMM
+    // when the shape rule in wq_gemm_ok does, else GEMV slices of 8 rows.
     const bool mfma = path == NQ_PATH_MFMA;
-    NQ_REQUIRE(!mfma || wq_gemm_ok(false, x, dtype_size(x_dtype), q, m, n, k, 32, ws != nullptr, true), NQ_BAD_ARG,
+    const bool operands = wq_gemm_ok(false, x, dtype_size(x_dtype), q, m, n, k, 32, ws != nullptr, true);
+    if (path == NQ_PATH_AUTO && wq_tile_route(false, x_dtype == NQ_F32, false, !fast && !long_k, !operands, m, n, k, 0, ws != nullptr))
+        return tile_gemm({x_dtype == NQ_F32 ? TileX::F32 : TileX::F16, x, reinterpret_cast<const uint8_t*>(q), false, w_scale,
+                          false, 0, nullptr, bias, y, y_dtype == NQ_F32 ? kTileF32 : kTileF16, m, n, k}, ws, ws_bytes, s);
+    NQ_REQUIRE(!mfma || operands, NQ_BAD_ARG,
                "linear_q8: the MFMA path needs k %% 32 == 0 and 16-byte aligned x and q (m=%lld n=%lld k=%lld)",
                (long long)m, (long long)n, (long long)k);
     if (mfma || (path == NQ_PATH_AUTO && wq_gemm_ok(false, x, dtype_size(x_dtype), q, m, n, k, 32, ws != nullptr))) {
@@ -2579,10 +2590,6 @@ nq_status linear_q8_impl(const void* x, nq_dtype x_dtype, const int8_t* q, const
             return wq_gemm<false>(static_cast<const _Float16*>(x), w, w_scale, bias, static_cast<float*>(y), m, n, k, 32, ws, ws_bytes, s);
         return wq_gemm<false>(static_cast<const _Float16*>(x), w, w_scale, bias, static_cast<_Float16*>(y), m, n, k, 32, ws, ws_bytes, s);
     }
-    const bool fast = path != NQ_PATH_GENERIC && k % 16 == 0 && k > 0 && k / 16 <= kMaxGemvThreads &&
-                      aligned(q, 16) && aligned(x, 16);
-    const bool long_k = path != NQ_PATH_GENERIC && k % 16 == 0 && k / 16 > kMaxGemvThreads && aligned(q, 16) &&
-                        aligned(x, 16);
     // Otherwise x rows beyond 8 run in slices of 8 (each slice re-streams the weight).
     for (int64_t r0 = 0; r0 < m; r0 += 8) {
         const int mi = static_cast<int>(m - r0 < 8 ? m - r0 : 8);
@@ -2636,10 +2643,19 @@ nq_status linear_q4g_impl(const void* x, nq_dtype x_dtype, const uint8_t* q, con
                NQ_BAD_ALIGN, "linear_q4g: misaligned pointer");
     hipStream_t s = as_stream(stream);
     const int ni = static_cast<int>(n), ki = static_cast<int>(k), gi = static_cast<int>(group);
-    // Batched activations: the fp16 MFMA GEMM when the shape rule in wq_gemm_ok
-    // picks it, else GEMV slices of 8 rows.
+    const bool aligned16 = aligned(q, 16) && aligned(x, 16);
+    const bool fast = path != NQ_PATH_GENERIC && k % 32 == 0 && k > 0 && group % 32 == 0 &&
+                      k / 32 <= kMaxGemvThreads && aligned16;
+    const bool long_k = path != NQ_PATH_GENERIC && k % 32 == 0 && group % 32 == 0 && k / 32 > kMaxGemvThreads && aligned16;
+    // Batched activations: the tile GEMM where wq_tile_route picks it, the MFMA GEMM
+    // when the shape rule in wq_gemm_ok does, else GEMV slices of 8 rows.
     const bool mfma = path == NQ_PATH_MFMA;
-    NQ_REQUIRE(!mfma || wq_gemm_ok(true, x, dtype_size(x_dtype), q, m, n, k, group, ws != nullptr, true), NQ_BAD_ARG,
+    const bool operands = wq_gemm_ok(true, x, dtype_size(x_dtype), q, m, n, k, group, ws != nullptr, true);
+    if (path == NQ_PATH_AUTO && wq_tile_route(true, x_dtype == NQ_F32, scale_dtype == NQ_F16, !fast && !long_k, !operands, m,
+                                              n, k, group, ws != nullptr))
+        return tile_gemm({x_dtype == NQ_F32 ? TileX::F32 : TileX::F16, x, q, true, scale, scale_dtype == NQ_F16, group, nullptr,
+                          bias, y, y_dtype == NQ_F32 ? kTileF32 : kTileF16, m, n, k}, ws, ws_bytes, s);
+    NQ_REQUIRE(!mfma || operands, NQ_BAD_ARG,
                "linear_q4g: the MFMA path needs k %% 32 == 0, group = 32 * 2^j and 16-byte aligned x and q "
                "(m=%lld n=%lld k=%lld group=%lld)", (long long)m, (long long)n, (long long)k, (long long)group);
     if (mfma || (path == NQ_PATH_AUTO && wq_gemm_ok(true, x, dtype_size(x_dtype), q, m, n, k, group, ws != nullptr))) {
@@ -2655,10 +2671,6 @@ nq_status linear_q4g_impl(const void* x, nq_dtype x_dtype, const uint8_t* q, con
         if (x_dtype == NQ_F32) return with_y(static_cast<const float*>(x));
         return with_y(static_cast<const _Float16*>(x));
     }
-    const bool fast = path != NQ_PATH_GENERIC && k % 32 == 0 && k > 0 && group % 32 == 0 &&
-                      k / 32 <= kMaxGemvThreads && aligned(q, 16) && aligned(x, 16);
-    const bool long_k = path != NQ_PATH_GENERIC && k % 32 == 0 && group % 32 == 0 && k / 32 > kMaxGemvThreads &&
-                        aligned(q, 16) && aligned(x, 16);
     for (int64_t r0 = 0; r0 < m; r0 += 8) {
         const int mi = static_cast<int>(m - r0 < 8 ? m - r0 : 8);
         const size_t xo = static_cast<size_t>(r0) * k, yo = static_cast<size_t>(r0) * n;
@@ -2706,6 +2718,11 @@ extern "C" nq_status nq_linear_q4g(const void* x, nq_dtype x_dtype, const uint8_
 
 extern "C" size_t nq_linear_wq_workspace_size(int64_t m, int64_t n, int64_t k) {
     return m > 0 && n > 0 && k > 0 && k <= kMaxIndex && n <= kMaxIndex ? wq_workspace_bytes(m, n, k) : 0;
+}
+
+extern "C" size_t nq_linear_wq_workspace_preferred(int64_t m, int64_t n, int64_t k) {
+    if (m <= 0 || n <= 0 || k <= 0 || k > kMaxIndex || n > kMaxIndex) return 0;
+    return std::max(wq_workspace_bytes(m, n, k), wq_tile_ws_bytes(m, n, k));
 }
 
 extern "C" nq_status nq_linear_q8_ws(const void* x, nq_dtype x_dtype, const int8_t* q, const float* w_scale,

@@ -24,6 +24,7 @@
 
 #include "nq_device.hpp"
 #include "nq_internal.hpp"
+#include "nq_tile_gemm.hpp"
 
 namespace nq {
 
@@ -808,11 +809,30 @@ int resolve_path(int path, int64_t m, int64_t n, int64_t k) {
                                                                                           : NQ_PATH_MFMA;
 }
 
+// Whether AUTO runs the tile GEMM (nq_tile_gemm.hip): from m = 9 where the operands fit
+// neither the MFMA kernels nor the GEMVs (k % 16, alignment; us, wave per row -> this:
+// m = 40, n = 1001, k = 1003 68 -> 8.2; m = 128, n = 4864, k = 900 264 -> 9.2), and past
+// 128 rows where k % 64 keeps the wide tiles away (the skinny kernel over 64-row
+// blocks: m = 1122, n = 1336, k = 5488 69 -> 32; 1.1x at m <= 512, 2.1x above). Its
+// int32 sums are exact, so the results are the other paths' bit for bit.
+bool w8a8_tile_route(bool operands_ok, int64_t m, int64_t n, int64_t k) {
+    if (!tile_gemm_ok(false, m, n, k, 0)) return false;
+    return operands_ok ? m > 128 && k % kBK != 0 : m >= 9;
+}
+size_t w8a8_tile_ws_bytes(int64_t m, int64_t n, int64_t k) {
+    if (!w8a8_tile_route(k > 0 && k % 16 == 0, m, n, k)) return 0;
+    return tile_gemm_ws_bytes(TileX::I8, false, m, n, k);
+}
+
 // Runs the chosen path on pre-quantized activations.
 nq_status run_gemm(const int8_t* xq, const float* as, const int8_t* wq, const float* ws,
                    const float* bias, void* y, nq_dtype ydt, int32_t* acc_out, int64_t m,
                    int64_t n, int64_t k, void* workspace, size_t ws_bytes, int path, hipStream_t s) {
     int p = resolve_path(path, m, n, k);
+    if (path == NQ_PATH_AUTO && w8a8_tile_route(mfma_ok(xq, wq, k), m, n, k))
+        return tile_gemm({TileX::I8, xq, reinterpret_cast<const uint8_t*>(wq), false, ws, false, 0, as, bias,
+                          acc_out ? acc_out : y, acc_out ? kTileI32 : ydt == NQ_F32 ? kTileF32 : kTileF16, m, n, k},
+                         workspace, ws_bytes, s);
     if (p == NQ_PATH_MFMA && !mfma_ok(xq, wq, k)) p = NQ_PATH_GENERIC;
     // Weights past 2^31 bytes exceed the MFMA kernels' 32-bit buffer offsets;
     // the v_dot4 GEMV (64-bit addressing) takes them, in slices of 8 rows.
@@ -912,6 +932,15 @@ extern "C" size_t nq_linear_w8a8_workspace_size(int64_t m, int64_t n, int64_t k)
            gemm_ws_bytes(m, n, k);
 }
 
+extern "C" size_t nq_gemm_w8a8_workspace_preferred(int64_t m, int64_t n, int64_t k) {
+    return std::max(gemm_ws_bytes(m, n, k), w8a8_tile_ws_bytes(m, n, k));
+}
+
+extern "C" size_t nq_linear_w8a8_workspace_preferred(int64_t m, int64_t n, int64_t k) {
+    if (m <= 0) return 0;
+    return nq_linear_w8a8_workspace_size(m, n, k) - gemm_ws_bytes(m, n, k) + nq_gemm_w8a8_workspace_preferred(m, n, k);
+}
+
 extern "C" nq_status nq_gemm_w8a8(const int8_t* xq, const float* a_scale, const int8_t* wq,
                                   const float* w_scale, const float* bias, void* y,
                                   nq_dtype y_dtype, int64_t m, int64_t n, int64_t k,
@@ -1005,7 +1034,7 @@ extern "C" nq_status nq_linear_w8a8(const void* x, nq_dtype x_dtype, const int8_
         nq_status st = NQ_OK;
         if (w8a8_decode_launch(xq, NQ_F16, wq, w_scale, bias, y, y_dtype, m, n, k, s, &st, as)) return st;
     }
-    return run_gemm(xq, as, wq, w_scale, bias, y, y_dtype, nullptr, m, n, k, rest, rest_bytes, p, s);
+    return run_gemm(xq, as, wq, w_scale, bias, y, y_dtype, nullptr, m, n, k, rest, rest_bytes, path, s);
 }
 
 // ---- the allocation-free W8A8 linear -------------------------------------------------------

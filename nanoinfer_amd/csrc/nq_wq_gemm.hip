@@ -28,11 +28,13 @@
 // reduced through LDS in wave order, so results are deterministic.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <iterator>
 #include <type_traits>
 
 #include "nq_device.hpp"
 #include "nq_internal.hpp"
+#include "nq_tile_gemm.hpp"
 
 namespace nq {
 namespace {
@@ -381,6 +383,13 @@ struct WqRowPlan {
     int tm, tn, splits, per;
 };
 
+// Split K of the 16-row kernel: up to 32 rows of x, and with fp32 x on weights of up to
+// 4096 rows from m = 17; the tile GEMM has the rest.
+template <typename XT>
+constexpr bool wq_row_split_built(int tm, int tn) {
+    return tm == 1 || (tm == 2 && (sizeof(XT) == 2 || tn == 1));
+}
+
 template <bool Q4, typename XT, typename YT, typename ST>
 nq_status launch_wq(const XT* x, const uint8_t* w, const ST* sc, const float* b, YT* y, int m, int n, int k,
                     int g, WqRowPlan p, float* planes, hipStream_t s) {
@@ -396,12 +405,15 @@ nq_status launch_wq(const XT* x, const uint8_t* w, const ST* sc, const float* b,
     auto go = [&](auto tmtag, auto tntag) {
         constexpr int TM = decltype(tmtag)::value, TN = decltype(tntag)::value;
         const dim3 grid(static_cast<unsigned>((n + 16 * TN - 1) / (16 * TN)), mblocks, static_cast<unsigned>(p.splits));
-        if (planes)
-            gemm_wq_kernel<Q4, TM, TN, XT, YT, ST, true><<<grid, wq_waves<TM>() * 64, 0, s>>>(x, w, sc, b, y, m, n, k,
-                                                                                             g, planes, p.per);
-        else
-            gemm_wq_kernel<Q4, TM, TN, XT, YT, ST><<<grid, wq_waves<TM>() * 64, 0, s>>>(x, w, sc, b, y, m, n, k, g,
-                                                                                       nullptr, p.per);
+        if constexpr (wq_row_split_built<XT>(TM, TN)) {
+            if (planes) {
+                gemm_wq_kernel<Q4, TM, TN, XT, YT, ST, true><<<grid, wq_waves<TM>() * 64, 0, s>>>(x, w, sc, b, y, m, n, k,
+                                                                                                 g, planes, p.per);
+                return;
+            }
+        }
+        gemm_wq_kernel<Q4, TM, TN, XT, YT, ST><<<grid, wq_waves<TM>() * 64, 0, s>>>(x, w, sc, b, y, m, n, k, g,
+                                                                                   nullptr, p.per);
     };
     auto with_tn = [&](auto tmtag) {
         if constexpr (decltype(tmtag)::value <= 2) {
@@ -806,7 +818,7 @@ nq_status launch_wq_wide(const XT* x, const uint8_t* w, const ST* sc, const floa
 // two 91.9, 256 x 128 in three 100).
 struct WqTile {
     int fm, fn, sk;
-    bool shallow = false;  // a two-slot ring (fm = 1, fn = 2 or 4): more workgroups per CU
+    bool shallow = false;  // a two-slot ring (fm = 1, fn = 2): more workgroups per CU
 };
 constexpr WqTile kWqTiles[] = {{4, 9, 64}, {4, 8, 64}, {2, 9, 128}, {4, 4, 64}, {2, 8, 128},
                                {2, 4, 128}, {1, 8, 128}, {1, 4, 128}, {1, 2, 128}};
@@ -876,7 +888,7 @@ nq_status wq_wide_tiles(const XT* x, const uint8_t* w, const ST* sc, const float
         constexpr int SK = decltype(skt)::value, FM = decltype(fmt)::value, FN2 = decltype(fnt)::value;
         constexpr int WN = Q4 ? 2 : FN2 % 3 == 0 ? 3 : FN2 % 4 == 0 ? 4 : 2, FN = FN2 * 2 / WN;
         using D8 = integral_constant<int, 8>;
-        if constexpr (FM == 1 && (FN2 == 2 || FN2 == 4)) {
+        if constexpr (!F32X && FM == 1 && FN2 == 2) {
             if (pick.shallow)  // two ring slots: two or three workgroups per CU
                 return launch_g(skt, fmt, integral_constant<int, FN>{}, integral_constant<int, WN>{},
                                 integral_constant<int, 4>{}, integral_constant<int, 2>{});
@@ -1045,6 +1057,12 @@ WqRoute plan_wq_route(int64_t m, int64_t n, int64_t k, bool wide_ok, bool wide_c
     r.per = p.per;
     return r;
 }
+// Whether a split route has its kernels here; the tile GEMM took the others over. Their
+// planes stay in the required workspace, whose size callers were given.
+template <typename XT>
+bool wq_split_built(const WqRoute& r) {
+    return r.wide ? sizeof(XT) == 2 && r.tile.fn == 2 : wq_row_split_built<XT>(r.row.tm, r.row.tn);
+}
 size_t wq_route_bytes(const WqRoute& r, int64_t m, int64_t n) {
     return r.splits > 1 ? round_up(static_cast<size_t>(r.splits) * static_cast<size_t>(m) * static_cast<size_t>(n) * 4, 256) : 0;
 }
@@ -1140,7 +1158,7 @@ nq_status wq_gemm(const XT* x, const uint8_t* w, const ST* sc, const float* b, Y
     const bool sk64 = wq_sk64_ok<Q4, ST>(group), f32x = sizeof(XT) == 4;
     const bool wide_ok = wq_wide_ok<Q4, XT, ST>(m, n, k, group), contract = wq_wide_contract<Q4, XT, ST>(m, n, k, group);
     WqRoute r = plan_wq_route(m, n, k, wide_ok, contract, sk64, f32x, workspace != nullptr, Q4);
-    if (r.splits > 1 && workspace_bytes < wq_route_bytes(r, m, n))
+    if (r.splits > 1 && (!wq_split_built<XT>(r) || workspace_bytes < wq_route_bytes(r, m, n)))
         r = plan_wq_route(m, n, k, wide_ok, contract, sk64, f32x, false, Q4);
     float* planes = r.splits > 1 ? static_cast<float*>(workspace) : nullptr;
     const int mi = static_cast<int>(m), ni = static_cast<int>(n), ki = static_cast<int>(k), gi = static_cast<int>(group);
@@ -1148,9 +1166,63 @@ nq_status wq_gemm(const XT* x, const uint8_t* w, const ST* sc, const float* b, Y
     return launch_wq<Q4>(x, w, sc, b, y, mi, ni, ki, gi, r.row, planes, s);
 }
 
+// Whether this call runs on the tile GEMM (nq_tile_gemm.hip) instead (us or factors
+// old -> new, measured over 1780 shapes):
+//   from m = 9 where no kernel here nor any GEMV takes the operands (`general`: k %
+//   16 or 32, alignment, groups), which fell to a wave per row (all of 250 shapes, 1.1 to
+//   10^4 times; m = 40, n = 1001, k = 1003: Q8 82 -> 8.8, Q4G 138 -> 8.9; m = 1500, n =
+//   6768, k = 2160: Q8 2146 -> 90, one int4 group per row 6 * 10^5 -> 88, a lane per group);
+//   from m = 16 where only the GEMVs do, in slices of 8 rows (`slices`; one int4 group per
+//   row, seldom a power of two of chunks, 10x), and for one group per row throughout,
+//   except fp16 x past m = 512 on the wide tiles' contract;
+//   fp32 x from m = 32 and k = 512 (2.8x; m = 333, n = 1536, k = 8960 Q8 85 -> 45), and from
+//   m = 16 on k >= 1024 and 512 weight rows (1.5x); shorter K loses up to 1.3x;
+//   fp16 x off the wide tiles' contract, or too few of them, from m = 33 and k = 1024
+//   (1.6x); on it from m = 65 and k = 1024 up to 1.5 Mi outputs (1.2x), and on more where
+//   they would split K (m = 584, n = 8125, k = 5888 Q4G 162 -> 138); else the wide tiles win
+//   (m = 2048, n = 8960, k = 1536 Q8 56 against 96).
+// A call without a workspace keeps the other kernels where the tiles want to split K.
+bool wq_tile_route(bool q4, bool f32x, bool scale_f16, bool general, bool slices, int64_t m, int64_t n, int64_t k,
+                   int64_t group, bool ws) {
+    if (!tile_gemm_ok(q4, m, n, k, group)) return false;
+    if (general) return m >= 9;
+    const bool row = q4 && group >= k;
+    bool wide;
+    if (!q4) wide = f32x ? wq_wide_contract<false, float, float>(m, n, k, 32) : wq_wide_contract<false, _Float16, float>(m, n, k, 32);
+    else if (f32x) wide = wq_wide_contract<true, float, float>(m, n, k, group);
+    else wide = scale_f16 ? wq_wide_contract<true, _Float16, _Float16>(m, n, k, group) : wq_wide_contract<true, _Float16, float>(m, n, k, group);
+    wide = wide && !slices;
+    if (m >= 16 && (slices || (row && (f32x || m <= 512 || !wide)))) return true;
+    bool take;
+    if (f32x) {
+        take = (m >= 32 && k >= 512) || (m >= 16 && k >= 1024 && n >= 512);
+    } else if (m < 33 || k < 1024) {
+        take = false;
+    } else if (!wide) {
+        take = true;
+    } else {
+        const bool sk64 = !q4 || group == 32;
+        const bool few = m <= 128 && plan_wq_wide(m, n, sk64, false).tiles < 128;  // no wide tiles unsplit
+        const WqRoute r = plan_wq_route(m, n, k, !few, true, sk64, false, ws, q4);
+        take = !r.wide || (m >= 65 && (r.splits > 1 || m * n <= (int64_t(3) << 19)));
+    }
+    return take && (ws || tile_gemm_split_fits(f32x ? TileX::F32 : TileX::F16, q4 && !row, m, n, k, 0));
+}
+
+// The split-K planes that the tile GEMM uses when the workspace holds them, for any
+// activation dtype and weight format that may take it at this shape.
+size_t wq_tile_ws_bytes(int64_t m, int64_t n, int64_t k) {
+    if (m < 9 || (m < 16 && k % 32 == 0) || !tile_gemm_ok(false, m, n, k, 0)) return 0;
+    size_t most = 0;
+    for (TileX xt : {TileX::F32, TileX::F16})
+        for (bool grouped : {false, true}) most = std::max(most, tile_gemm_ws_bytes(xt, grouped, m, n, k));
+    return most;
+}
+
 // Workspace the split-K planes take at this shape (0: no split): the most any
 // activation dtype or group size can plan, so one size serves every call.
 size_t wq_workspace_bytes(int64_t m, int64_t n, int64_t k) {
+    if (k < 32) return 0;  // no whole chunk to split
     if (m <= 0 || n <= 0 || k <= 0 || !(wq_gemm_shape_ok(m, n, k, 2, true) || wq_q4_batch5_shape(m, n, k) ||
                                                    wq_q8_batch5_shape(m, n, k))) return 0;
     size_t most = 0;

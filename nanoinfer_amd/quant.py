@@ -257,7 +257,7 @@ def linear_q8(x: torch.Tensor, w: QTensor, bias=None, out_dtype=None, path: int 
     b = _bias(bias, w.out)
     y = torch.empty((x.shape[0], w.out), dtype=out_dtype or x.dtype, device=x.device)
     lib = _lib.load()
-    nbytes = lib.nq_linear_wq_workspace_size(x.shape[0], w.out, w.in_)
+    nbytes = lib.nq_linear_wq_workspace_preferred(x.shape[0], w.out, w.in_)
     ws = _workspace(nbytes, x.device) if nbytes else None
     check(lib.nq_linear_q8_ex(_ptr(x), _dtype_code(x, "x"), _ptr(w.q), _ptr(w.scale), _ptr(b), _ptr(y),
                               _dtype_code(y, "y"), x.shape[0], w.out, w.in_, _ptr(ws), nbytes, int(path),
@@ -273,7 +273,7 @@ def linear_q4g(x: torch.Tensor, w: Q4GTensor, bias=None, out_dtype=None, path: i
     b = _bias(bias, w.out)
     y = torch.empty((x.shape[0], w.out), dtype=out_dtype or x.dtype, device=x.device)
     lib = _lib.load()
-    nbytes = lib.nq_linear_wq_workspace_size(x.shape[0], w.out, w.in_)
+    nbytes = lib.nq_linear_wq_workspace_preferred(x.shape[0], w.out, w.in_)
     ws = _workspace(nbytes, x.device) if nbytes else None
     check(lib.nq_linear_q4g_ex(_ptr(x), _dtype_code(x, "x"), _ptr(w.q), _ptr(w.scale),
                                _dtype_code(w.scale, "scale"), w.group, _ptr(b), _ptr(y), _dtype_code(y, "y"),
@@ -365,7 +365,7 @@ def linear_w8a8(x: torch.Tensor, w: QTensor, bias=None, out_dtype=None, path: in
     lib = _lib.load()
     m = x.shape[0]
     y = torch.empty((m, w.out), dtype=out_dtype or x.dtype, device=x.device)
-    nbytes = lib.nq_linear_w8a8_workspace_size(m, w.out, w.in_)
+    nbytes = lib.nq_linear_w8a8_workspace_preferred(m, w.out, w.in_)
     ws = _workspace(nbytes, x.device)
     check(lib.nq_linear_w8a8(_ptr(x), _dtype_code(x, "x"), _ptr(w.q), _ptr(w.scale), _ptr(b), _ptr(y),
                              _dtype_code(y, "y"), m, w.out, w.in_, _ptr(ws), ws.numel(), path, _stream()))
@@ -380,7 +380,7 @@ def gemm_w8a8(xq, a_scale, w: QTensor, bias=None, out_dtype=torch.float16, path:
     b = _bias(bias, w.out)
     lib = _lib.load()
     y = torch.empty((m, w.out), dtype=out_dtype, device=xq.device)
-    ws = _workspace(lib.nq_gemm_w8a8_workspace_size(m, w.out, w.in_), xq.device)
+    ws = _workspace(lib.nq_gemm_w8a8_workspace_preferred(m, w.out, w.in_), xq.device)
     check(lib.nq_gemm_w8a8(_ptr(xq), _ptr(a_scale), _ptr(w.q), _ptr(w.scale), _ptr(b), _ptr(y),
                            _dtype_code(y, "y"), m, w.out, w.in_, _ptr(ws), ws.numel(), path, _stream()))
     return y
@@ -396,7 +396,7 @@ def w8a8_acc_i32(xq: torch.Tensor, wq: torch.Tensor, path: int = NQ_PATH_AUTO) -
     n = wq.shape[0]
     lib = _lib.load()
     acc = torch.empty((m, n), dtype=torch.int32, device=xq.device)
-    ws = _workspace(lib.nq_gemm_w8a8_workspace_size(m, n, k), xq.device)
+    ws = _workspace(lib.nq_gemm_w8a8_workspace_preferred(m, n, k), xq.device)
     check(lib.nq_w8a8_acc_i32(_ptr(xq), _ptr(wq), _ptr(acc), m, n, k, _ptr(ws), ws.numel(), path, _stream()))
     return acc
 

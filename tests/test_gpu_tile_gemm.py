@@ -1,0 +1,153 @@
+"""The tile GEMM (any k, alignment and group of whole chunks) through the public linears,
+against float64 on the device at the edges of its tiles, slabs and split plans, and
+against the wave-per-row kernels (NQ_PATH_GENERIC) on the same operands."""
+import numpy as np
+import pytest
+import torch
+
+from test_spills import _spills
+
+F16, F32 = torch.float16, torch.float32
+gpu = pytest.mark.gpu
+
+
+def _codes(t, group):
+    """Dequantized weights in float64 from the packed bytes."""
+    if group == 0:
+        return t.q.double() * t.scale.double()[:, None]
+    nib = torch.stack([t.q & 15, t.q >> 4], 2).reshape(t.out, -1)[:, :t.in_].double() - 8
+    return nib * t.scale.double().repeat_interleave(group, 1)[:, :t.in_]
+
+
+def _make(nq, fmt, n, k, group, sdt, g):
+    w = torch.randn(n, k, generator=g, device="cuda") * 0.02
+    if fmt == "q8":
+        return nq.quantize_q8(w), 0
+    return (nq.quantize_q4g(w, group, sdt), group) if fmt == "q4g" else (nq.quantize_q4(w), max(1, k))
+
+
+def _check(y, x, wd, b, k):
+    """Any order of fp32 sums of exact products (three bf16 parts for fp32 x) is within
+    3 k 2^-24 sum|x w|; scale, bias and the fp16 store round a few times more."""
+    ref = x.double() @ wd.t().contiguous()
+    lim = 3 * k * 2.0 ** -24 * (x.double().abs() @ wd.abs().t().contiguous())
+    if b is not None:
+        ref, lim = ref + b.double(), lim + 2.0 ** -22 * b.double().abs()
+    lim = lim + 2.0 ** -21 * ref.abs()
+    if y.dtype == F16:
+        lim = lim + 2.0 ** -10 * ref.abs() + 2.0 ** -24
+    assert y.shape == ref.shape
+    assert bool(((y.double() - ref).abs() <= lim).all())
+    if y.dtype == F32:  # the bound is loose by sqrt(k): measured 1e-7 on all plans
+        assert float((y.double() - ref).norm() / ref.norm()) < 2e-6
+
+
+# one shape per tile and plan (whole and split K), k off every slab, odd n and m; then
+# k below a chunk and a slab, exact slabs, one row of weights
+PLANS = [(9, 65, 65), (9, 65, 2051), (400, 65, 2051), (700, 65, 1003), (33, 515, 2051), (130, 6001, 65),
+         (257, 6001, 131), (257, 2003, 1003), (700, 515, 2051), (257, 4001, 1003), (520, 4001, 515), (777, 8960, 500),
+         (1000, 4001, 325), (5, 1, 7), (9, 33, 31), (17, 130, 33), (64, 64, 320), (65, 129, 129), (16, 600, 1024)]
+
+
+@gpu
+@pytest.mark.parametrize("xdt", [F32, F16])
+@pytest.mark.parametrize("fmt,group", [("q8", 0), ("q4", 0), ("q4g", 32), ("q4g", 96), ("q4g", 128), ("q4g", 4096)])
+def test_linear(dev, nq, xdt, fmt, group):
+    g = torch.Generator(device=dev).manual_seed(group + len(fmt))
+    for i, (m, n, k) in enumerate(PLANS):
+        t, gr = _make(nq, fmt, n, k, group, F16 if i % 2 else F32, g)
+        x = torch.randn(m, k, generator=g, device=dev).to(xdt)
+        b = torch.randn(n, generator=g, device=dev) if i % 3 else None
+        y = (nq.linear_q8 if fmt == "q8" else nq.linear_q4g)(x, t, b, F16 if i % 4 == 3 else F32)
+        _check(y, x, _codes(t, gr), b, k)
+
+
+@gpu
+@pytest.mark.parametrize("m,n,k", PLANS + [(300, 200, 1040), (1122, 136, 5488), (16, 150, 1500), (520, 6001, 2051)])
+def test_w8a8_exact(dev, nq, m, n, k):
+    from nanoinfer_amd import _lib
+    g = torch.Generator(device=dev).manual_seed(m + n + k)
+    xq = torch.randint(-127, 128, (m, k), generator=g, device=dev, dtype=torch.int8)
+    wq = torch.randint(-127, 128, (n, k), generator=g, device=dev, dtype=torch.int8)
+    acc = nq.w8a8_acc_i32(xq, wq)
+    assert torch.equal(acc.double(), xq.double() @ wq.double().t().contiguous())  # sums below 2^53
+    t = nq.QTensor(wq, torch.rand(n, generator=g, device=dev) * 1e-3, n, k)
+    a_s, b = torch.rand(m, generator=g, device=dev), torch.randn(n, generator=g, device=dev)
+    for ydt in (F32, F16):
+        got = nq.gemm_w8a8(xq, a_s, t, b, ydt)
+        ref = nq.gemm_w8a8(xq, a_s, t, b, ydt, path=_lib.NQ_PATH_GENERIC)
+        assert torch.equal(got, ref)
+
+
+@gpu
+@pytest.mark.parametrize("xdt", [F32, F16])
+def test_misaligned_rows_and_nonfinite_values(dev, nq, xdt):
+    """Row starts off every alignment (views one element in), and infinities and NaN, which
+    stay in their row and agree with the wave-per-row kernel."""
+    from nanoinfer_amd import _lib
+    g = torch.Generator(device=dev).manual_seed(3)
+    for m, n, k in ((21, 70, 256), (40, 130, 259)):
+        buf = torch.randn(m * k + 1, generator=g, device=dev).to(xdt)
+        x = buf[1:].view(m, k)
+        x[3, k - 1], x[5, 0], x[7, 40] = float("inf"), float("nan"), -float("inf")
+        for t, f in ((nq.quantize_q8(torch.randn(n, k, generator=g, device=dev)), nq.linear_q8),
+                     (nq.quantize_q4g(torch.randn(n, k, generator=g, device=dev), 32), nq.linear_q4g)):
+            y, ref = f(x, t, None, F32), f(x, t, None, F32, path=_lib.NQ_PATH_GENERIC)
+            assert torch.equal(torch.isnan(y), torch.isnan(ref)) and torch.equal(torch.isinf(y), torch.isinf(ref))
+            rows = torch.ones(m, dtype=torch.bool, device=dev)
+            rows[[3, 5, 7]] = False
+            assert bool(torch.isfinite(y[rows]).all())
+            assert float((y[rows] - ref[rows]).norm() / ref[rows].norm()) < 2e-6
+
+
+# What stays with the kernels of 16 rows and 64-row split tiles: short K and fp32 x, few
+# rows of x on a wide weight, fp16 x up to 64 rows (unsplit, split, and all output types).
+KEPT = [(F32, 20, 300, 96), (F32, 40, 130, 160), (F32, 100, 130, 160), (F32, 20, 130, 2080), (F32, 12, 5000, 4128),
+        (F32, 25, 4200, 160), (F16, 40, 300, 160), (F16, 100, 4200, 96), (F16, 24, 130, 2080), (F16, 40, 300, 2048),
+        (F16, 24, 4200, 4128)]
+
+
+@gpu
+@pytest.mark.parametrize("xdt,m,n,k", KEPT)
+@pytest.mark.parametrize("fmt,sdt", [("q8", F32), ("q4g", F32), ("q4g", F16)])
+def test_neighbours_of_the_route(dev, nq, xdt, m, n, k, fmt, sdt):
+    g = torch.Generator(device=dev).manual_seed(m + n)
+    t, gr = _make(nq, fmt, n, k, 32, sdt, g)
+    x = torch.randn(m, k, generator=g, device=dev).to(xdt)
+    for ydt in (F32, F16):
+        _check((nq.linear_q8 if fmt == "q8" else nq.linear_q4g)(x, t, None, ydt), x, _codes(t, gr), None, k)
+
+
+@gpu
+def test_less_workspace_splits_less(dev, nq):
+    """The plain entries (no workspace) and a workspace below the preferred size give the
+    same result up to the order of the sums."""
+    from nanoinfer_amd import _lib
+    lib, m, n, k = _lib.load(), 70, 600, 2019
+    best = lib.nq_linear_wq_workspace_preferred(m, n, k)
+    assert best >= 2 * m * n * 4 and lib.nq_linear_wq_workspace_size(m, n, k) == 0
+    t = nq.quantize_q8(torch.randn(n, k, device=dev))
+    x = torch.randn(m, k, device=dev)
+    full = nq.linear_q8(x, t)
+    ws = torch.empty(best, dtype=torch.uint8, device=dev)
+    y = torch.empty_like(full)
+    for nbytes in (0, m * n * 4, best // 2):
+        y.fill_(-1)
+        _lib.check(lib.nq_linear_q8_ws(x.data_ptr(), 0, t.q.data_ptr(), t.scale.data_ptr(), None, y.data_ptr(), 0, m, n, k,
+                                       ws.data_ptr() if nbytes else None, nbytes, torch.cuda.current_stream().cuda_stream))
+        assert float((y - full).norm() / full.norm()) < 1e-6
+
+
+def test_workspace_sizes_of_short_k():
+    """Shapes below one 32-column chunk: no workspace is required (a division by the
+    number of chunks once stood here)."""
+    from nanoinfer_amd import _lib
+    lib = _lib.load()
+    for m in (1, 9, 64, 300):
+        for k in (1, 7, 31):
+            assert lib.nq_linear_wq_workspace_size(m, 100, k) == 0
+            assert lib.nq_linear_wq_workspace_preferred(m, 100, k) % 256 == 0
+
+
+def test_no_spills():
+    assert not {k: v for k, v in _spills("nq_tile_gemm.hip").items() if v}
