@@ -2574,9 +2574,12 @@ nq_status linear_q8_impl(const void* x, nq_dtype x_dtype, const int8_t* q, const
     // when the shape rule in wq_gemm_ok does, else GEMV slices of 8 rows.
     const bool mfma = path == NQ_PATH_MFMA;
     const bool operands = wq_gemm_ok(false, x, dtype_size(x_dtype), q, m, n, k, 32, ws != nullptr, true);
-    if (path == NQ_PATH_AUTO && wq_tile_route(false, x_dtype == NQ_F32, false, !fast && !long_k, !operands, m, n, k, 0, ws != nullptr))
-        return tile_gemm({x_dtype == NQ_F32 ? TileX::F32 : TileX::F16, x, reinterpret_cast<const uint8_t*>(q), false, w_scale,
-                          false, 0, nullptr, bias, y, y_dtype == NQ_F32 ? kTileF32 : kTileF16, m, n, k}, ws, ws_bytes, s);
+    const bool general = !fast && !long_k;
+    const TileCall tile{x_dtype == NQ_F32 ? TileX::F32 : TileX::F16, x, reinterpret_cast<const uint8_t*>(q), false, w_scale,
+                        false, 0, nullptr, bias, y, y_dtype == NQ_F32 ? kTileF32 : kTileF16, m, n, k};
+    if (path == NQ_PATH_AUTO && general && m <= 8 && tile_gemm_ok(false, m, n, k, 0)) return gemv_any(tile, s);
+    if (path == NQ_PATH_AUTO && wq_tile_route(false, x_dtype == NQ_F32, false, general, !operands, m, n, k, 0, ws != nullptr))
+        return tile_gemm(tile, ws, ws_bytes, s);
     NQ_REQUIRE(!mfma || operands, NQ_BAD_ARG,
                "linear_q8: the MFMA path needs k %% 32 == 0 and 16-byte aligned x and q (m=%lld n=%lld k=%lld)",
                (long long)m, (long long)n, (long long)k);
@@ -2651,10 +2654,13 @@ nq_status linear_q4g_impl(const void* x, nq_dtype x_dtype, const uint8_t* q, con
     // when the shape rule in wq_gemm_ok does, else GEMV slices of 8 rows.
     const bool mfma = path == NQ_PATH_MFMA;
     const bool operands = wq_gemm_ok(true, x, dtype_size(x_dtype), q, m, n, k, group, ws != nullptr, true);
-    if (path == NQ_PATH_AUTO && wq_tile_route(true, x_dtype == NQ_F32, scale_dtype == NQ_F16, !fast && !long_k, !operands, m,
-                                              n, k, group, ws != nullptr))
-        return tile_gemm({x_dtype == NQ_F32 ? TileX::F32 : TileX::F16, x, q, true, scale, scale_dtype == NQ_F16, group, nullptr,
-                          bias, y, y_dtype == NQ_F32 ? kTileF32 : kTileF16, m, n, k}, ws, ws_bytes, s);
+    const bool general = !fast && !long_k;
+    const TileCall tile{x_dtype == NQ_F32 ? TileX::F32 : TileX::F16, x, q, true, scale, scale_dtype == NQ_F16, group, nullptr,
+                        bias, y, y_dtype == NQ_F32 ? kTileF32 : kTileF16, m, n, k};
+    if (path == NQ_PATH_AUTO && general && m <= 8 && tile_gemm_ok(true, m, n, k, group)) return gemv_any(tile, s);
+    if (path == NQ_PATH_AUTO && wq_tile_route(true, x_dtype == NQ_F32, scale_dtype == NQ_F16, general, !operands, m, n, k,
+                                              group, ws != nullptr))
+        return tile_gemm(tile, ws, ws_bytes, s);
     NQ_REQUIRE(!mfma || operands, NQ_BAD_ARG,
                "linear_q4g: the MFMA path needs k %% 32 == 0, group = 32 * 2^j and 16-byte aligned x and q "
                "(m=%lld n=%lld k=%lld group=%lld)", (long long)m, (long long)n, (long long)k, (long long)group);

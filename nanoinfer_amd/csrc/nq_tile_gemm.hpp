@@ -32,4 +32,7 @@ size_t tile_gemm_ws_bytes(TileX xt, bool grouped, int64_t m, int64_t n, int64_t 
 bool tile_gemm_split_fits(TileX xt, bool grouped, int64_t m, int64_t n, int64_t k, size_t ws_bytes);
 nq_status tile_gemm(const TileCall& c, void* ws, size_t ws_bytes, hipStream_t s);
 
+// The same operands at m <= 8 (nq_gemv_any.hip); no workspace.
+nq_status gemv_any(const TileCall& c, hipStream_t s);
+
 }  // namespace nq

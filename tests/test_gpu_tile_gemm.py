@@ -48,6 +48,11 @@ PLANS = [(9, 65, 65), (9, 65, 2051), (400, 65, 2051), (700, 65, 1003), (33, 515,
          (257, 6001, 131), (257, 2003, 1003), (700, 515, 2051), (257, 4001, 1003), (520, 4001, 515), (777, 8960, 500),
          (1000, 4001, 325), (5, 1, 7), (9, 33, 31), (17, 130, 33), (64, 64, 320), (65, 129, 129), (16, 600, 1024)]
 
+# the GEMVs of up to 8 rows: M buckets, pieces of 8 and 16 columns and their partial last
+# one, K over 1, 2 and 4 waves, two and four weight rows per wave, ragged row counts
+GEMVS = [(1, 1, 1), (1, 67, 15), (2, 130, 33), (3, 131, 1003), (8, 70, 1003), (5, 9, 8), (1, 515, 2051), (2, 70, 4099),
+         (4, 66, 4099), (7, 67, 8191), (1, 8193, 259), (2, 8194, 131), (3, 8195, 67), (8, 8197, 131)]
+
 
 @gpu
 @pytest.mark.parametrize("xdt", [F32, F16])
@@ -63,7 +68,7 @@ def test_linear(dev, nq, xdt, fmt, group):
 
 
 @gpu
-@pytest.mark.parametrize("m,n,k", PLANS + [(300, 200, 1040), (1122, 136, 5488), (16, 150, 1500), (520, 6001, 2051)])
+@pytest.mark.parametrize("m,n,k", PLANS + GEMVS + [(300, 200, 1040), (1122, 136, 5488), (16, 150, 1500), (520, 6001, 2051)])
 def test_w8a8_exact(dev, nq, m, n, k):
     from nanoinfer_amd import _lib
     g = torch.Generator(device=dev).manual_seed(m + n + k)
@@ -81,12 +86,25 @@ def test_w8a8_exact(dev, nq, m, n, k):
 
 @gpu
 @pytest.mark.parametrize("xdt", [F32, F16])
+@pytest.mark.parametrize("fmt,group", [("q8", 0), ("q4", 0), ("q4g", 32), ("q4g", 96)])
+def test_gemv(dev, nq, xdt, fmt, group):
+    g = torch.Generator(device=dev).manual_seed(group + len(fmt))
+    for i, (m, n, k) in enumerate(GEMVS):
+        t, gr = _make(nq, fmt, n, k, group, F16 if i % 2 else F32, g)
+        x = torch.randn(m, k, generator=g, device=dev).to(xdt)
+        b = torch.randn(n, generator=g, device=dev) if i % 3 else None
+        y = (nq.linear_q8 if fmt == "q8" else nq.linear_q4g)(x, t, b, F16 if i % 4 == 3 else F32)
+        _check(y, x, _codes(t, gr), b, k)
+
+
+@gpu
+@pytest.mark.parametrize("xdt", [F32, F16])
 def test_misaligned_rows_and_nonfinite_values(dev, nq, xdt):
     """Row starts off every alignment (views one element in), and infinities and NaN, which
     stay in their row and agree with the wave-per-row kernel."""
     from nanoinfer_amd import _lib
     g = torch.Generator(device=dev).manual_seed(3)
-    for m, n, k in ((21, 70, 256), (40, 130, 259)):
+    for m, n, k in ((8, 33, 256), (8, 20, 259), (21, 70, 256), (40, 130, 259)):
         buf = torch.randn(m * k + 1, generator=g, device=dev).to(xdt)
         x = buf[1:].view(m, k)
         x[3, k - 1], x[5, 0], x[7, 40] = float("inf"), float("nan"), -float("inf")
@@ -150,4 +168,5 @@ def test_workspace_sizes_of_short_k():
 
 
 def test_no_spills():
-    assert not {k: v for k, v in _spills("nq_tile_gemm.hip").items() if v}
+    for src in ("nq_tile_gemm.hip", "nq_gemv_any.hip"):
+        assert not {k: v for k, v in _spills(src).items() if v}
