@@ -75,11 +75,23 @@ def _host_artifacts():
           "-I", sysconfig.get_paths()["include"], "-o", mod + ".tmp", os.path.join(host_src, "nicpp.cpp"),
           "-L", PKG, "-lnq_host", "-lnq_hip", rpath], "nicpp module")
     os.replace(mod + ".tmp", mod)
+    # _calls: the native call path of quant.py, on torch's own tensors and allocator.
+    import torch
+
+    troot = os.path.dirname(torch.__file__)
+    calls = os.path.join(PKG, "_calls" + ext)
+    _run([*cxx, "-shared", "-fvisibility=hidden", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", os.path.join(troot, "include"),
+          "-I", os.path.join(troot, "include", "torch", "csrc", "api", "include"),
+          "-I", sysconfig.get_paths()["include"], "-o", calls + ".tmp", os.path.join(host_src, "nq_calls.cpp"),
+          "-L", PKG, "-lnq_hip", "-L", os.path.join(troot, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", rpath],
+         "_calls module")
+    os.replace(calls + ".tmp", calls)
     _run([*cxx, "-o", HOST_TEST + ".tmp", os.path.join(ROOT, "tests", "cpp", "test_host.cpp"),
           "-L", PKG, "-lnq_host", "-lnq_hip", "-Wl,-rpath," + PKG, "-Wl,-rpath,$ORIGIN/../../nanoinfer_amd"],
          "C++ host test")
     os.replace(HOST_TEST + ".tmp", HOST_TEST)
-    return [HOST_LIB, mod, HOST_TEST]
+    return [HOST_LIB, mod, calls, HOST_TEST]
 
 
 def build(verbose: bool = False) -> str:

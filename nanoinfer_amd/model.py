@@ -115,6 +115,9 @@ def apply_rope(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.T
 def rope_qkv(qkv: torch.Tensor, heads: int, kv_heads: int, head_dim: int, cos: torch.Tensor, sin: torch.Tensor):
     """One launch for the fused q|k|v output [s, (heads + 2 kv) d]: RoPE on q and
     k (ops.cpp:145-166) and all three written head-major [h, s, d]."""
+    r = quant._calls.rope_qkv(qkv, heads, kv_heads, head_dim, cos, sin)
+    if r is not None:
+        return r
     from ._lib import check, load
     s = qkv.shape[0]
     if qkv.stride(1) != 1 or cos.dtype != torch.float32 or cos.shape[0] < s:
@@ -259,7 +262,8 @@ class Model:
             x, *xq = quant.add_rmsnorm_quant(x, o, self.norm[L + "post_attention_layernorm"], cfg.eps)
             gu = self.gemm(tuple(xq), L + "mlp.gate_up_proj")
             i = cfg.intermediate
-            return x, self.gemm(quant.silu_mul_quant(gu[:, :i], gu[:, i:]), L + "mlp.down_proj")
+            act = quant._calls.silu_mul_quant(gu, None) or quant.silu_mul_quant(gu[:, :i], gu[:, i:])
+            return x, self.gemm(act, L + "mlp.down_proj")
         a = a.transpose(0, 1).reshape(s, hq).contiguous()
         x = x + self.project(a, L + "self_attn.o_proj")
         hm = rmsnorm(x, self.norm[L + "post_attention_layernorm"], cfg.eps)

@@ -21,6 +21,11 @@ from ._lib import NQ_F16, NQ_F32, NQ_PATH_AUTO, check
 
 _lib.load()  # fail loudly at import when the HIP library is missing
 
+# Each operation first asks the native call path, which takes plain calls whole
+# (contiguous device tensors of the expected types and shapes) and returns None for
+# every other; what follows it here converts, or raises.
+from . import _calls  # noqa: E402
+
 _DT = {torch.float32: NQ_F32, torch.float16: NQ_F16}
 
 
@@ -131,6 +136,9 @@ def _w2d(w, who):
 
 def quantize_q8(w: torch.Tensor) -> QTensor:
     """quant.cpp:88-108 (device side, bit-exact)."""
+    r = _calls.quantize(w, 0, None)
+    if r is not None:
+        return QTensor(r[0], r[1], *r[0].shape)
     w = _w2d(w, "quantize_q8")
     out, k = w.shape
     q = torch.empty((out, k), dtype=torch.int8, device=w.device)
@@ -141,6 +149,10 @@ def quantize_q8(w: torch.Tensor) -> QTensor:
 
 def quantize_q4g(w: torch.Tensor, group: int = 32, scale_dtype=torch.float32) -> Q4GTensor:
     """quant.cpp:295-321 (device side, bit-exact codes; fp16 scale storage optional)."""
+    if isinstance(group, int) and group > 0:
+        r = _calls.quantize(w, group, scale_dtype)
+        if r is not None:
+            return Q4GTensor(r[0], r[1], *w.shape, group)
     w = _w2d(w, "quantize_q4g")
     if group <= 0:
         raise ValueError("quantize_q4g: group must be positive")
@@ -161,6 +173,9 @@ def quantize_q4(w: torch.Tensor) -> Q4GTensor:
 
 def act_quant(x: torch.Tensor):
     """The activation quant of linear_w8a8 (quant.cpp:179-193): (xq int8, a_scale fp32)."""
+    r = _calls.act_quant(x)
+    if r is not None:
+        return r
     x = _dev(x, "x")
     if x.dim() != 2:
         raise ValueError("act_quant expects 2-D x")
@@ -174,6 +189,9 @@ def act_quant(x: torch.Tensor):
 def act_quant_heads(a: torch.Tensor):
     """act_quant of a head-major [heads, s, d] tensor's transpose [s, heads*d]
     (an attention output feeding o_proj) without the transpose copy."""
+    r = _calls.act_quant_heads(a)
+    if r is not None:
+        return r
     a = _dev(a, "a")
     if a.dim() != 3 or not a.is_contiguous():
         raise ValueError("act_quant_heads expects a contiguous [heads, s, d] tensor")
@@ -187,6 +205,9 @@ def act_quant_heads(a: torch.Tensor):
 def rmsnorm_quant(x: torch.Tensor, w: torch.Tensor, eps: float):
     """rmsnorm (ops.cpp:272-290) with the act quant of linear_w8a8 fused in:
     (xq int8, a_scale fp32) of x * (1/sqrt(mean(x^2) + eps)) * w."""
+    r = _calls.rmsnorm_quant(x, w, eps)
+    if r is not None:
+        return r
     x = _dev(x, "x")
     if x.dim() != 2:
         raise ValueError("rmsnorm_quant expects 2-D x")
@@ -204,6 +225,10 @@ def rmsnorm_quant(x: torch.Tensor, w: torch.Tensor, eps: float):
 def add_rmsnorm_quant(x: torch.Tensor, r: torch.Tensor, w: torch.Tensor, eps: float, inplace: bool = False):
     """h = x + r (the residual add, model.cpp:175-186) and rmsnorm_quant(h) in one
     launch: returns (h, xq, a_scale); with inplace=True h is written into x."""
+    if not inplace:
+        y = _calls.add_rmsnorm_quant(x, r, w, eps)
+        if y is not None:
+            return y
     x, r = _dev(x, "x"), _dev(r, "r")
     if x.dim() != 2 or r.shape != x.shape or r.dtype != x.dtype or not x.is_contiguous() or not r.is_contiguous():
         raise ValueError("add_rmsnorm_quant: x and r must be contiguous 2-D tensors of one shape and dtype")
@@ -223,6 +248,10 @@ def silu_mul_quant(gate: torch.Tensor, up: torch.Tensor):
     """silu(gate) * up (ops.cpp:86-100) with the act quant fused in. gate and up
     are [m, k] views with unit column stride and one common row stride (e.g. the
     two halves of a fused gate|up projection output)."""
+    if up is not None:
+        r = _calls.silu_mul_quant(gate, up)
+        if r is not None:
+            return r
     if not (isinstance(gate, torch.Tensor) and gate.is_cuda and isinstance(up, torch.Tensor) and up.is_cuda):
         raise ValueError("gate and up must be device tensors")
     if gate.shape != up.shape or gate.dim() != 2 or gate.dtype != up.dtype:
@@ -252,6 +281,9 @@ def linear_q8(x: torch.Tensor, w: QTensor, bias=None, out_dtype=None, path: int 
     allocator. path forces a kernel family (the per-call form of the
     reference's CudaPolicy::force_tiled_q8, cuda_backend.hpp:57-59):
     NQ_PATH_GEMV, NQ_PATH_MFMA or NQ_PATH_GENERIC (nq_linear_q8_ex)."""
+    y = _calls.linear(0, x, w.q, w.scale, bias, out_dtype, w.out, w.in_, 0, path)
+    if y is not None:
+        return y
     w.check()
     x = _x2d(x, w.in_, "linear_q8")
     b = _bias(bias, w.out)
@@ -268,6 +300,9 @@ def linear_q8(x: torch.Tensor, w: QTensor, bias=None, out_dtype=None, path: int 
 def linear_q4g(x: torch.Tensor, w: Q4GTensor, bias=None, out_dtype=None, path: int = NQ_PATH_AUTO) -> torch.Tensor:
     """quant.cpp:337-389 (no GPU counterpart in the reference); split K and
     the per-call path as linear_q8 (nq_linear_q4g_ex)."""
+    y = _calls.linear(1, x, w.q, w.scale, bias, out_dtype, w.out, w.in_, w.group, path)
+    if y is not None:
+        return y
     w.check()
     x = _x2d(x, w.in_, "linear_q4g")
     b = _bias(bias, w.out)
@@ -359,6 +394,9 @@ def _workspace(nbytes: int, device) -> torch.Tensor:
 
 def linear_w8a8(x: torch.Tensor, w: QTensor, bias=None, out_dtype=None, path: int = NQ_PATH_AUTO):
     """quant.cpp:165-210 / cuda_quant.cu:250-284."""
+    y = _calls.linear(2, x, w.q, w.scale, bias, out_dtype, w.out, w.in_, 0, path)
+    if y is not None:
+        return y
     w.check()
     x = _x2d(x, w.in_, "linear_w8a8")
     b = _bias(bias, w.out)
@@ -374,6 +412,9 @@ def linear_w8a8(x: torch.Tensor, w: QTensor, bias=None, out_dtype=None, path: in
 
 def gemm_w8a8(xq, a_scale, w: QTensor, bias=None, out_dtype=torch.float16, path: int = NQ_PATH_AUTO):
     """W8A8 on pre-quantized activations (the GEMM half of cuda_linear_w8a8)."""
+    y = _calls.gemm_w8a8(xq, a_scale, w.q, w.scale, bias, out_dtype, w.out, w.in_, path)
+    if y is not None:
+        return y
     w.check()
     xq = _dev(xq, "xq")
     m = xq.shape[0]
