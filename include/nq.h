@@ -166,6 +166,12 @@ nq_status nq_silu_mul_f32(const float* gate, const float* up, int64_t ld, int64_
 nq_status nq_attention_causal_f32(const float* q, const float* k, const float* v, int64_t heads, int64_t kv_heads,
                                   int64_t s, int64_t head_dim, float* out, void* stream);
 
+/* The same on fp16 heads with fp32 scores, softmax and sums (the weights enter the second
+ * product in fp16): q [heads, s, d], k / v [kv_heads, s, d], out [heads, s, d] head-major,
+ * head_dim 64 or 128, 16-byte aligned. */
+nq_status nq_attention_causal_f16(const void* q, const void* k, const void* v, int64_t heads, int64_t kv_heads, int64_t s,
+                                  int64_t head_dim, void* out, void* stream);
+
 /* ---- weight files: quantize on load -------------------------------------------
  * NIT0 / NIT1 files (serialize.hpp:1-23; load_bin serialize.cpp:11-72): the same
  * header checks as load_bin (bad magic, unknown dtype, negative ndim or dim,

@@ -58,6 +58,7 @@ SIGNATURES = {
     "nq_rmsnorm_f32": (_D, [_P, _P, _P, _P, ctypes.c_float, _I, _I, _P, _P]),
     "nq_silu_mul_f32": (_D, [_P, _P, _I, _I, _I, _P, _P]),
     "nq_attention_causal_f32": (_D, [_P, _P, _P, _I, _I, _I, _I, _P, _P]),
+    "nq_attention_causal_f16": (_D, [_P, _P, _P, _I, _I, _I, _I, _P, _P]),
     "nq_nit_info": (_D, [ctypes.c_char_p, _P, _P, _P, ctypes.c_int32]),
     "nq_nit_load_f32": (_D, [ctypes.c_char_p, _P, _I, _P]),
     "nq_nit_load_q8": (_D, [ctypes.c_char_p, _P, _P, _I, _I, _P]),

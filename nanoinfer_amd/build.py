@@ -23,7 +23,7 @@ HOST_TEST = os.path.join(ROOT, "tests", "cpp", "test_host.bin")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-SOURCES = ["nq_abi.cpp", "nq_quantize.hip", "nq_gemv.hip", "nq_w8a8.hip", "nq_embed.hip", "nq_fused.hip", "nq_wq_gemm.hip", "nq_tile_gemm.hip", "nq_gemv_any.hip", "nq_nit.hip", "nq_rope.hip", "nq_dequant.hip", "nq_ops.hip"]
+SOURCES = ["nq_abi.cpp", "nq_quantize.hip", "nq_gemv.hip", "nq_w8a8.hip", "nq_embed.hip", "nq_fused.hip", "nq_wq_gemm.hip", "nq_tile_gemm.hip", "nq_gemv_any.hip", "nq_attention.hip", "nq_nit.hip", "nq_rope.hip", "nq_dequant.hip", "nq_ops.hip"]
 BENCH_SRC = os.path.join("bench", "nq_probe.hip")  # libnq_bench.so: bench.py's read probe
 BENCH_LIB = os.path.join(PKG, "libnq_bench.so")
 

@@ -10,6 +10,7 @@
 // allocator reports an error: the caller then runs its Python path, which converts what
 // it accepts and raises what it refuses.
 #include <ATen/ATen.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
@@ -273,6 +274,27 @@ PyObject* rope_qkv(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
+// attention(q [heads, s, d], k, v [kv, s, d]) -> [heads, s, d], causal, fp16 heads of 64 or
+// 128. It stands where a differentiable torch call stands otherwise, so it declines
+// whatever autograd, forward mode or a dispatch mode could want to see.
+PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    return call<3>(n, [&](int dev, hipStream_t s) -> PyObject* {
+        In q, k, v;
+        if (c10::impl::TorchDispatchModeTLS::any_modes_set() || !q.packed(a[0], dev) || !k.packed(a[1], dev) || !v.packed(a[2], dev))
+            return nullptr;
+        for (const In* t : {&q, &k, &v})
+            if (t->t->dim() != 3 || t->t->scalar_type() != at::kHalf || t->t->unsafeGetTensorImpl()->autograd_meta() != nullptr)
+                return nullptr;
+        const int64_t h = q.size(0), rows = q.size(1), d = q.size(2), kv = k.size(0);
+        if ((d != 64 && d != 128) || k.t->sizes() != v.t->sizes() || k.size(1) != rows || k.size(2) != d || kv < 1 || h < 1 || h % kv ||
+            rows > (d == 64 ? 1024 : 2048))  // measured up to here: longer rows are torch's
+            return nullptr;
+        const at::Tensor out = empty({h, rows, d}, at::kHalf, dev);
+        const bool ok = launch([&] { return nq_attention_causal_f16(q.p(), k.p(), v.p(), h, kv, rows, d, out.data_ptr(), s); });
+        return ok ? wrap(out) : nullptr;
+    });
+}
+
 // quantize(w, group, scale_dtype) -> (codes, scales); group 0: int8 per row
 PyObject* quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return call<3>(n, [&](int dev, hipStream_t s) -> PyObject* {
@@ -295,7 +317,7 @@ PyObject* quantize(PyObject*, PyObject* const* a, Py_ssize_t n) {
 
 #define NQ_CALL(f) {#f, reinterpret_cast<PyCFunction>(reinterpret_cast<void*>(f)), METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {NQ_CALL(linear), NQ_CALL(gemm_w8a8), NQ_CALL(act_quant), NQ_CALL(act_quant_heads), NQ_CALL(rmsnorm_quant),
-                         NQ_CALL(add_rmsnorm_quant), NQ_CALL(silu_mul_quant), NQ_CALL(rope_qkv), NQ_CALL(quantize),
+                         NQ_CALL(add_rmsnorm_quant), NQ_CALL(silu_mul_quant), NQ_CALL(rope_qkv), NQ_CALL(attention), NQ_CALL(quantize),
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_calls", "Native call path of nanoinfer_amd.quant.", -1, methods, nullptr, nullptr, nullptr, nullptr};
 

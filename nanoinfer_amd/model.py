@@ -133,9 +133,14 @@ def rope_qkv(qkv: torch.Tensor, heads: int, kv_heads: int, head_dim: int, cos: t
 
 def attention(q, k, v, n_rep: int) -> torch.Tensor:
     """ops.cpp:206-270: causal softmax(q k^T / sqrt(d)) v with the KV heads
-    repeated n_rep times (GQA); scores and softmax in fp32. fp16 activations use
-    torch's fused scaled-dot-product attention (fp32 softmax inside)."""
+    repeated n_rep times (GQA); scores and softmax in fp32. fp16 heads of 64 or 128
+    run on the library's kernel; other fp16 ones, and tensors that autograd follows,
+    on torch's fused scaled-dot-product attention (fp32 softmax inside)."""
     if q.dtype == torch.float16:
+        if q.dim() == 3 and q.shape[0] == k.shape[0] * n_rep:
+            a = quant._calls.attention(q, k, v)
+            if a is not None:
+                return a
         return torch.nn.functional.scaled_dot_product_attention(
             q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), is_causal=True, enable_gqa=n_rep > 1).squeeze(0)
     k = k.repeat_interleave(n_rep, 0)
