@@ -18,7 +18,7 @@ constexpr int kRowThreads = 256;
 
 // One workgroup per row: absmax over the row (block reduction through LDS),
 // scale = absmax / 127, then each thread quantizes its strided elements.
-// Used for weights (quantize_q8) and activations (W8A8 act quant).
+// Rows that the vector kernel below does not take (fewer than 8 elements, or over 65536).
 template <typename XT>
 __global__ __launch_bounds__(kRowThreads) void quantize_rows_i8_kernel(
     const XT* __restrict__ x, int8_t* __restrict__ q, float* __restrict__ scale, int k) {
@@ -76,23 +76,38 @@ __global__ void quantize_q4g_even_kernel(const float* __restrict__ w, uint8_t* _
     }
 }
 
-// Vector path (group = 8 G with G a power of two <= 64, in % 8 == 0): lane t
-// owns 8 consecutive columns (two 16-byte loads) of a row whose chunks are
-// padded to a multiple of G, so the G lanes of one block are an aligned run of
-// a wave; the block absmax is a G-lane shuffle reduction (order-free), and the
-// lane writes its 4 packed bytes with one 32-bit store. Lanes past the row's
-// end (a partial last block) contribute 0 to the absmax and store nothing.
-template <typename ST, int G>
-__global__ __launch_bounds__(256) void quantize_q4g_vec_kernel(const float* __restrict__ w, uint32_t* __restrict__ q,
+// Vector path (group = 8 G with G a power of two <= 64): lane t owns 8 consecutive
+// columns (two 16-byte loads, at whatever address the row starts) of a row whose
+// chunks are padded to a multiple of G, so the G lanes of one block are an aligned run
+// of a wave; the block absmax is a G-lane shuffle reduction (order-free), and the lane
+// writes its 4 packed bytes with one 32-bit store. Lanes past the row's end (a partial
+// last block) contribute 0 to the absmax and store nothing; the lane of a partial
+// last chunk (in % 8) reads and writes it column by column (ANY; without it, for whole
+// aligned chunks, n = 17920, k = 1536 takes 23.2 us and not 23.5).
+// Rows off 8 columns took a thread per block with strided scalar loads: n = 9000, k =
+// 9001, groups of 32 2746 -> 71 us (5.2 TB/s).
+template <typename ST, int G, bool ANY>
+__global__ __launch_bounds__(256) void quantize_q4g_vec_kernel(const float* __restrict__ w, uint8_t* __restrict__ q,
                                                                ST* __restrict__ scale, int out, int in, int blocks,
                                                                int cpr) {
     const int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
     const bool live = t < static_cast<int64_t>(out) * cpr;
     const int o = live ? static_cast<int>(t / cpr) : 0, cc = live ? static_cast<int>(t % cpr) : 0;
     const bool act = live && cc * 8 < in;
-    const f4* src = reinterpret_cast<const f4*>(w + static_cast<size_t>(o) * in + (act ? cc * 8 : 0));
-    const f4 a = src[0], b = src[1];
-    const float v[8] = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    const int cols = act ? min(in - cc * 8, 8) : 0;
+    const float* src = w + static_cast<size_t>(o) * in + (act ? cc * 8 : 0);
+    float v[8];
+    if constexpr (!ANY) {
+        __builtin_memcpy(v, __builtin_assume_aligned(src, 16), 32);
+    } else if (cols == 8) {
+        __builtin_memcpy(v, src, 32);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const float f = src[max(min(j, cols - 1), 0)];
+            v[j] = j < cols ? f : 0.0f;
+        }
+    }
     float am = 0.0f;
 #pragma unroll
     for (int j = 0; j < 8; ++j) am = absmax_step(am, v[j]);
@@ -109,7 +124,15 @@ __global__ __launch_bounds__(256) void quantize_q4g_vec_kernel(const float* __re
         const uint32_t hi = static_cast<uint32_t>(static_cast<int>(rq.code(v[2 * j + 1], 7.0f)) + 8);
         word |= (lo | (hi << 4)) << (8 * j);
     }
-    q[static_cast<size_t>(o) * (in / 8) + cc] = word;
+    uint8_t* dst = q + static_cast<size_t>(o) * ((in + 1) / 2) + static_cast<size_t>(cc) * 4;
+    if constexpr (!ANY) {
+        __builtin_memcpy(__builtin_assume_aligned(dst, 4), &word, 4);
+    } else if (cols == 8) {
+        __builtin_memcpy(dst, &word, 4);
+    } else {
+        if (cols & 1) word &= ~(0xF0u << (4 * (cols - 1)));  // the odd last column's high nibble stays 0
+        for (int j = 0; j < (cols + 1) / 2; ++j) dst[j] = static_cast<uint8_t>(word >> (8 * j));
+    }
 }
 
 // Odd group: one thread per packed byte; each of its two columns recomputes its
@@ -139,8 +162,11 @@ __global__ void quantize_q4g_odd_kernel(const float* __restrict__ w, uint8_t* __
 }
 
 // ---- activation quant (vectorized) ------------------------------
-// One workgroup per row, 8 elements per 16-byte step held in registers between
-// the absmax pass and the quantize pass (x is read once).
+// One workgroup per row, 8 elements per 16-byte step (fp16) held in registers between
+// the absmax pass and the quantize pass (x is read once), at whatever address the row
+// starts; the last k % 8 elements go one to a thread. Rows off 8 elements took two
+// passes of single elements (us: m = 2048, k = 1003 fp16 8.3 -> 7.3; m = 512, k = 8955
+// 16.5 -> 8.7; weights of 9000 x 9001 181 -> 75).
 // HEADS: x is head-major [k / hd, m, hd] (an attention output) and row `row`
 // is the concatenation of its heads' row-`row` segments, i.e. the rows of the
 // [m, k] matrix its transpose would produce (hd = 8 * epr elements per head).
@@ -150,19 +176,18 @@ __global__ __launch_bounds__(NT) void act_quant_vec_kernel(const XT* __restrict_
     __shared__ float red[NT / 64];
     const int tid = threadIdx.x;
     typedef XT v8 __attribute__((ext_vector_type(8)));
-    const int row = blockIdx.x, steps = k >> 3;
-    const v8* xr = reinterpret_cast<const v8*>(x + static_cast<size_t>(row) * (HEADS ? 8 * epr : k));
+    const int row = blockIdx.x, steps = k >> 3, rest = HEADS ? 0 : k & 7;
+    const XT* xr = x + static_cast<size_t>(row) * (HEADS ? 8 * epr : k);
     v8 v[CPT];
-    float am = 0.0f;
+    const XT lone = tid < rest ? xr[8 * steps + tid] : static_cast<XT>(0.0f);
+    float am = absmax_step(0.0f, to_f32(lone));
     // Loads are unconditional (indices past the row re-read its last vector and
     // are left out of the absmax), so all CPT of them are in flight together.
 #pragma unroll
     for (int c = 0; c < CPT; ++c) {
         const int e = min(tid + c * NT, steps - 1);
-        if constexpr (HEADS)
-            v[c] = xr[static_cast<size_t>(e / epr) * m * epr + e % epr];
-        else
-            v[c] = xr[e];
+        const size_t at = HEADS ? static_cast<size_t>(e / epr) * m * epr + e % epr : static_cast<size_t>(e);
+        __builtin_memcpy(&v[c], xr + 8 * at, sizeof(v8));
     }
     __builtin_amdgcn_sched_barrier(0);  // keep every load ahead of the absmax math
 #pragma unroll
@@ -182,7 +207,8 @@ __global__ __launch_bounds__(NT) void act_quant_vec_kernel(const XT* __restrict_
     if (tid == 0) a_scale[row] = sc;
     const RowQuantizer rq(sc);
     typedef int v2i __attribute__((ext_vector_type(2)));
-    v2i* qr = reinterpret_cast<v2i*>(xq + static_cast<size_t>(row) * k);
+    int8_t* qr = xq + static_cast<size_t>(row) * k;
+    if (tid < rest) qr[8 * steps + tid] = static_cast<int8_t>(rq.code(to_f32(lone), 127.0f));
 #pragma unroll
     for (int c = 0; c < CPT; ++c) {
         const int e = tid + c * NT;
@@ -193,7 +219,8 @@ __global__ __launch_bounds__(NT) void act_quant_vec_kernel(const XT* __restrict_
                 lo |= (static_cast<int>(rq.code(to_f32(v[c][j]), 127.0f)) & 0xFF) << (8 * j);
                 hi |= (static_cast<int>(rq.code(to_f32(v[c][j + 4]), 127.0f)) & 0xFF) << (8 * j);
             }
-            qr[e] = v2i{lo, hi};
+            const v2i both = {lo, hi};
+            __builtin_memcpy(qr + 8 * static_cast<size_t>(e), &both, 8);
         }
     }
 }
@@ -215,7 +242,7 @@ nq_status act_quant(const void* x, nq_dtype xdt, int64_t m, int64_t k, int8_t* x
     // One workgroup per row: for m >= 256, 256 threads with up to 8 vectors of
     // 8 elements each (k <= 16384; several vectors per thread keep more loads
     // in flight and let several rows share a CU), else 1024 threads with up to 8.
-    const bool vec = k > 0 && k % 8 == 0 && k <= 8 * 1024 * 8 && aligned(x, 16) && aligned(xq, 8);
+    const bool vec = k >= 8 && k <= 8 * 1024 * 8;
     if (vec) {
         const unsigned grid = static_cast<unsigned>(m);
         const int64_t steps = k / 8;
@@ -337,13 +364,16 @@ extern "C" nq_status nq_quantize_q4g(const float* w, int64_t out, int64_t in, in
     const int threads = 256;
     hipStream_t s = as_stream(stream);
     const int gl = g / 8;  // lanes per block on the vector path
-    if (g % 8 == 0 && gl <= 64 && (gl & (gl - 1)) == 0 && k % 8 == 0 && aligned(w, 16) && aligned(q, 4)) {
-        const int cpr = ((k / 8 + gl - 1) / gl) * gl;
+    if (g % 8 == 0 && gl <= 64 && (gl & (gl - 1)) == 0) {
+        const int cpr = (((k + 7) / 8 + gl - 1) / gl) * gl;
         const unsigned grid = static_cast<unsigned>((out * cpr + 255) / 256);
         auto go = [&](auto gtag, auto* sp) {
             constexpr int G = decltype(gtag)::value;
             using ST = std::remove_pointer_t<decltype(sp)>;
-            quantize_q4g_vec_kernel<ST, G><<<grid, 256, 0, s>>>(w, reinterpret_cast<uint32_t*>(q), sp, o, k, blocks, cpr);
+            if (k % 8 == 0 && aligned(w, 16) && aligned(q, 4))
+                quantize_q4g_vec_kernel<ST, G, false><<<grid, 256, 0, s>>>(w, q, sp, o, k, blocks, cpr);
+            else
+                quantize_q4g_vec_kernel<ST, G, true><<<grid, 256, 0, s>>>(w, q, sp, o, k, blocks, cpr);
         };
         auto with_g = [&](auto* sp) {
             switch (gl) {

@@ -97,6 +97,20 @@ def test_gemv(dev, nq, xdt, fmt, group):
         _check(y, x, _codes(t, gr), b, k)
 
 
+# the wave-per-row kernels stay behind an explicit path, over every type they take
+@gpu
+@pytest.mark.parametrize("ydt", [F32, F16])
+@pytest.mark.parametrize("xdt", [F32, F16])
+def test_explicit_generic_path(dev, nq, xdt, ydt):
+    from nanoinfer_amd import _lib
+    g = torch.Generator(device=dev).manual_seed(5)
+    x, b = torch.randn(3, 203, generator=g, device=dev).to(xdt), torch.randn(65, generator=g, device=dev)
+    for fmt, group, sdt in (("q8", 0, F32), ("q4g", 32, F32), ("q4g", 32, F16)):
+        t, group = _make(nq, fmt, 65, 203, group, sdt, g)
+        f = nq.linear_q8 if fmt == "q8" else nq.linear_q4g
+        _check(f(x, t, b, out_dtype=ydt, path=_lib.NQ_PATH_GENERIC), x, _codes(t, group), b, 203)
+
+
 @gpu
 @pytest.mark.parametrize("xdt", [F32, F16])
 def test_misaligned_rows_and_nonfinite_values(dev, nq, xdt):
