@@ -354,12 +354,17 @@ __global__ __launch_bounds__((WM * WN * 64)) void tile_gemm_kernel(TileArgs a) {
     };
 
     // Sums in two levels, as one chain over all of K rounds its running sum once per MFMA:
-    // fp32 activations start each chunk's three products from zero, smallest part
-    // first, and `part` holds the sums of 256 columns or of the open group. The larger
-    // fp32 tiles on row scales add each chunk to the sum itself: `part` costs them
+    // fp32 activations start each chunk's three products from zero, largest part
+    // first, and `part` holds the sums of 256 columns or of the open group. (Smallest
+    // first is as good on one linear but leaves a mean error: the MFMA cuts the low
+    // bits of the sum it is given when larger products join, always downwards, m = 384,
+    // n = 896, k = 4864 -7.7e-8 of the rms against -1e-9, and a decoder's attention
+    // averages over such a shift without shrinking it: 2 layers, 384 tokens, int4 logits
+    // 6.5e-7 off and not 3.6e-7. Adding the largest part's product separately costs 5%.)
+    // The larger fp32 tiles on row scales add each chunk to the sum itself: `part` costs them
     // the second workgroup of a CU (m = 333, n = 1536, k = 8960 47 -> 54 us). Relative
-    // errors against 64 bits, K whole, one chain -> this: Q8 fp32 k = 1536 3.7e-7 ->
-    // 1.4e-7, fp16 k = 8960 5.7e-7 -> 1.4e-7; Q4G fp16 k = 4096 2.0e-7 -> 0.8e-7.
+    // errors against 64 bits, K whole, one chain -> this: Q8 fp32 k = 896 2.9e-7 ->
+    // 1.0e-7, fp16 k = 8960 5.7e-7 -> 1.4e-7; Q4G fp16 k = 4096 2.0e-7 -> 0.8e-7.
     constexpr bool PART = !I8 && (!BF || GROUPED || FN * FM <= 4);
     // Q4G closes a part with its group's scale; the others add it as it is.
     constexpr bool GSCALE = F == WF::Q4G;
@@ -404,7 +409,7 @@ __global__ __launch_bounds__((WM * WN * 64)) void tile_gemm_kernel(TileArgs a) {
                         Acc d = Acc{0, 0, 0, 0};
                         if constexpr (BF) {
 #pragma unroll
-                            for (int p = 2; p >= 0; --p)
+                            for (int p = 0; p < 3; ++p)
                                 d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(b8, xa[p][j]),
                                                                             __builtin_bit_cast(b8, wb[i]), d, 0, 0, 0);
                         } else {
