@@ -10,11 +10,14 @@
 // allocator reports an error: the caller then runs its Python path, which converts what
 // it accepts and raises what it refuses.
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Dtype.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include "../../../include/nq.h"
 
@@ -274,13 +277,22 @@ PyObject* rope_qkv(PyObject*, PyObject* const* a, Py_ssize_t n) {
     });
 }
 
+// Whether something besides the kernel wants to see or steer a torch call: a tracer, a
+// dispatch or torch-function mode, autocast, or a selection among torch's own attentions.
+bool torch_call_observed() {
+    const at::Context& c = at::globalContext();
+    return torch::jit::tracer::isTracing() || c10::impl::TorchDispatchModeTLS::any_modes_set() ||
+           at::impl::torch_function_mode_enabled() || at::autocast::is_autocast_enabled(at::kCUDA) ||
+           !(c.userEnabledFlashSDP() && c.userEnabledMemEfficientSDP() && c.userEnabledMathSDP());
+}
+
 // attention(q [heads, s, d], k, v [kv, s, d]) -> [heads, s, d], causal, fp16 heads of 64 or
 // 128. It stands where a differentiable torch call stands otherwise, so it declines
-// whatever autograd, forward mode or a dispatch mode could want to see.
+// whatever autograd or forward mode follows, and every call that torch_call_observed.
 PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return call<3>(n, [&](int dev, hipStream_t s) -> PyObject* {
         In q, k, v;
-        if (c10::impl::TorchDispatchModeTLS::any_modes_set() || !q.packed(a[0], dev) || !k.packed(a[1], dev) || !v.packed(a[2], dev))
+        if (torch_call_observed() || !q.packed(a[0], dev) || !k.packed(a[1], dev) || !v.packed(a[2], dev))
             return nullptr;
         for (const In* t : {&q, &k, &v})
             if (t->t->dim() != 3 || t->t->scalar_type() != at::kHalf || t->t->unsafeGetTensorImpl()->autograd_meta() != nullptr)

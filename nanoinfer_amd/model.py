@@ -134,10 +134,11 @@ def rope_qkv(qkv: torch.Tensor, heads: int, kv_heads: int, head_dim: int, cos: t
 def attention(q, k, v, n_rep: int) -> torch.Tensor:
     """ops.cpp:206-270: causal softmax(q k^T / sqrt(d)) v with the KV heads
     repeated n_rep times (GQA); scores and softmax in fp32. fp16 heads of 64 or 128
-    run on the library's kernel; other fp16 ones, and tensors that autograd follows,
-    on torch's fused scaled-dot-product attention (fp32 softmax inside)."""
+    run on the library's kernel; other fp16 ones, tensors that autograd follows, and
+    calls that a tracer, compiler, mode or autocast has to see, on torch's fused
+    scaled-dot-product attention (fp32 softmax inside)."""
     if q.dtype == torch.float16:
-        if q.dim() == 3 and q.shape[0] == k.shape[0] * n_rep:
+        if q.dim() == 3 and q.shape[0] == k.shape[0] * n_rep and not torch.compiler.is_compiling():
             a = quant._calls.attention(q, k, v)
             if a is not None:
                 return a

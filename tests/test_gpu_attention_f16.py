@@ -70,6 +70,44 @@ def test_calls_that_stay_with_torch(dev):
     assert qg.grad is not None and float((y.detach() - model.attention(q, k, v, 2)).abs().max()) < 4e-3
 
 
+class _Seen(torch.overrides.TorchFunctionMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        self.names.append(getattr(func, "__name__", ""))
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d", [64, 128])
+def test_traced_and_steered_calls_stay_with_torch(dev, d):
+    from nanoinfer_amd import model, quant
+    from torch.nn.attention import SDPBackend, sdpa_kernel
+    a, b = _inputs(4, 2, 33, d, 5, dev), _inputs(4, 2, 33, d, 6, dev)
+    call = lambda q, k, v: model.attention(q, k, v, 2)
+    traced = torch.jit.trace(call, a, check_trace=False)
+    assert "scaled_dot_product_attention" in str(traced.graph)
+    # both within the kernels' rounding of the other: 2^-11 of the values' size, a few times
+    assert float((traced(*b).float() - call(*b).float()).abs().max()) < 4e-3
+    with _Seen() as seen:
+        call(*a)
+    assert "scaled_dot_product_attention" in seen.names
+    with sdpa_kernel(SDPBackend.MATH):
+        assert quant._calls.attention(*a) is None
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert quant._calls.attention(*a) is None
+    assert quant._calls.attention(*a) is not None
+
+
+def test_compiles_as_one_graph():
+    from nanoinfer_amd import model
+    a = _inputs(4, 2, 20, 64, 7, "cpu")
+    f = torch.compile(lambda q, k, v: model.attention(q, k, v, 2), backend="eager", fullgraph=True)
+    assert torch.equal(f(*a), model.attention(*a, 2))
+
+
 @pytest.mark.gpu
 def test_inside_a_graph(dev):
     from nanoinfer_amd import model
