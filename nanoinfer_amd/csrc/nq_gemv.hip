@@ -2576,7 +2576,7 @@ nq_status linear_q8_impl(const void* x, nq_dtype x_dtype, const int8_t* q, const
     const bool operands = wq_gemm_ok(false, x, dtype_size(x_dtype), q, m, n, k, 32, ws != nullptr, true);
     const bool general = !fast && !long_k;
     const TileCall tile{x_dtype == NQ_F32 ? TileX::F32 : TileX::F16, x, reinterpret_cast<const uint8_t*>(q), false, w_scale,
-                        false, 0, nullptr, bias, y, y_dtype == NQ_F32 ? kTileF32 : kTileF16, m, n, k};
+                        false, 0, nullptr, bias, y, y_dtype == NQ_F32 ? kTileF32 : kTileF16, m, n, k, !operands};
     if (path == NQ_PATH_AUTO && general && m <= 8 && tile_gemm_ok(false, m, n, k, 0)) return gemv_any(tile, s);
     if (path == NQ_PATH_AUTO && wq_tile_route(false, x_dtype == NQ_F32, false, general, !operands, m, n, k, 0, ws != nullptr))
         return tile_gemm(tile, ws, ws_bytes, s);
@@ -2656,7 +2656,7 @@ nq_status linear_q4g_impl(const void* x, nq_dtype x_dtype, const uint8_t* q, con
     const bool operands = wq_gemm_ok(true, x, dtype_size(x_dtype), q, m, n, k, group, ws != nullptr, true);
     const bool general = !fast && !long_k;
     const TileCall tile{x_dtype == NQ_F32 ? TileX::F32 : TileX::F16, x, q, true, scale, scale_dtype == NQ_F16, group, nullptr,
-                        bias, y, y_dtype == NQ_F32 ? kTileF32 : kTileF16, m, n, k};
+                        bias, y, y_dtype == NQ_F32 ? kTileF32 : kTileF16, m, n, k, true};
     if (path == NQ_PATH_AUTO && general && m <= 8 && tile_gemm_ok(true, m, n, k, group)) return gemv_any(tile, s);
     if (path == NQ_PATH_AUTO && wq_tile_route(true, x_dtype == NQ_F32, scale_dtype == NQ_F16, general, !operands, m, n, k,
                                               group, ws != nullptr))

@@ -5,10 +5,11 @@
 //
 // A wave owns R weight rows and all M activation rows; its lanes take whole pieces of
 // PC columns (16-byte loads at any byte address) over K, which KW waves of the
-// workgroup share when the weight is too narrow to fill the GPU with rows. Pieces are
-// summed as the element kernel's order allows: fp32 FMAs per lane, then over the wave
-// in a fixed tree; int8 activations in int32 by v_dot4. The columns of the last, partial
-// piece are read one by one by a single lane, so nothing past a row is touched.
+// workgroup share when the weight is too narrow to fill the GPU with rows. A piece is
+// summed by fp32 FMAs, the pieces of a lane and then of the wave, in a fixed tree, in
+// fp64 (in fp32 they were off by 7.3e-8 where the element kernel's groups of 256 were by
+// 5.4e-8, k = 1003, fp16; now 2.6e-8); int8 activations in int32 by v_dot4. The columns of
+// the last, partial piece go one to a lane, so nothing past a row is touched.
 //
 // Bound by latency on small weights and by the activation re-reads (one per R weight
 // rows) at 8 rows. us, element kernel -> this: Q8 fp32 x, n = 1001, k = 1003 m = 7 15.4 ->
@@ -61,7 +62,7 @@ __global__ __launch_bounds__(256) void gemv_any_kernel(AnyArgs a) {
     constexpr int PC = I8 || M <= 2 ? 16 : 8;  // columns per piece: 8 keeps M rows of x in registers
     constexpr int WD = PC / (Q4 ? 8 : 4);      // dwords of a weight piece
     constexpr int NV = M * R;
-    using Acc = std::conditional_t<I8, int, float>;
+    using Acc = std::conditional_t<I8, int, double>;
     __shared__ Acc part[4][NV];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -96,10 +97,11 @@ __global__ __launch_bounds__(256) void gemv_any_kernel(AnyArgs a) {
 #pragma unroll
                 for (int d = 0; d < WD; ++d) acc[i * R + r] = __builtin_amdgcn_sdot4(w[r][d], xv[d], acc[i * R + r], false);
             } else {
-                float p = F == WF::Q4G ? 0.0f : acc[i * R + r];
+                float p = 0.0f;
 #pragma unroll
                 for (int e = 0; e < PC; ++e) p = __builtin_fmaf(xv[e], code(w[r], e), p);
-                acc[i * R + r] = F == WF::Q4G ? __builtin_fmaf(p, sc[r], acc[i * R + r]) : p;
+                if constexpr (F == WF::Q4G) acc[i * R + r] = __builtin_fma(static_cast<double>(p), static_cast<double>(sc[r]), acc[i * R + r]);
+                else acc[i * R + r] += p;
             }
         }
     };
@@ -124,21 +126,18 @@ __global__ __launch_bounds__(256) void gemv_any_kernel(AnyArgs a) {
             }
         }
     }
-    if (whole * PC < k && wk * 64 + lane == whole % (64 * kw)) {  // the lane whose turn the partial piece is
-        const int c = whole * PC;
+    if (wk == 0 && lane < k - whole * PC) {  // the partial piece, a column per lane
+        const int c = whole * PC + lane;
         float sc[R];
         scales(c, sc);
-        for (int e = 0; c + e < k; ++e) {
 #pragma unroll
-            for (int r = 0; r < R; ++r) {
-                const int b = Q4 ? wr[r][(c + e) >> 1] : wr[r][c + e];
-                const int q = Q4 ? (((c + e) & 1) ? b >> 4 : b & 15) - 8 : static_cast<int8_t>(b);
+        for (int r = 0; r < R; ++r) {
+            const int b = Q4 ? wr[r][c >> 1] : wr[r][c];
+            const int q = Q4 ? (c & 1 ? b >> 4 : b & 15) - 8 : static_cast<int8_t>(b);
 #pragma unroll
-                for (int i = 0; i < M; ++i) {
-                    if constexpr (I8) acc[i * R + r] += q * static_cast<int>(xr[i][c + e]);
-                    else if constexpr (F == WF::Q4G) acc[i * R + r] = __builtin_fmaf(to_f32(xr[i][c + e]) * static_cast<float>(q), sc[r], acc[i * R + r]);
-                    else acc[i * R + r] = __builtin_fmaf(to_f32(xr[i][c + e]), static_cast<float>(q), acc[i * R + r]);
-                }
+            for (int i = 0; i < M; ++i) {
+                if constexpr (I8) acc[i * R + r] += q * static_cast<int>(xr[i][c]);
+                else acc[i * R + r] += static_cast<double>(xr[i][c]) * q * (F == WF::Q4G ? sc[r] : 1.0f);
             }
         }
     }
@@ -164,8 +163,7 @@ __global__ __launch_bounds__(256) void gemv_any_kernel(AnyArgs a) {
     const float b = a.bias ? a.bias[row] : 0.0f;
     float t;
     if constexpr (I8) t = w8a8_epilogue(sum, a.a_scale[i], scale_at(a, row), b);
-    else if constexpr (F == WF::Q4G) t = sum + b;
-    else t = __builtin_fmaf(sum, scale_at(a, row), b);
+    else t = static_cast<float>(F == WF::Q4G ? sum + b : sum * scale_at(a, row) + b);
     if (a.y_kind == kTileF16) static_cast<_Float16*>(a.y)[o] = from_f32<_Float16>(t);
     else static_cast<float*>(a.y)[o] = t;
 }

@@ -19,9 +19,9 @@
 // past k as zeros, and that slab goes first, so that its latency hides behind the
 // first whole slabs. Rows past m or n are loaded as the last row and not stored.
 //
-// Results: products are exact in fp32 and sums are fp32 (int32 for int8) as in the
-// other MFMA kernels; int4 group sums are scaled by their group scale in fp32.
-// With K split over gridDim.y each range stores its raw sums into its own plane.
+// Results: products are exact in fp32; sums over up to 256 columns are fp32, and those
+// of K fp64 or fp32 (int32 for int8), see PART and FINE. With K split over gridDim.y
+// each range stores its raw sums into its own plane, in fp32.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -37,11 +37,13 @@ namespace {
 
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef __bf16 b8 __attribute__((ext_vector_type(8)));
+typedef double d4 __attribute__((ext_vector_type(4)));
 
-// Weight formats: int8 codes, int4 codes with one scale per row, int4 in groups
-// of 32 columns, int4 in groups of a larger multiple of 32.
-enum class WF { Q8, Q4Row, Q4G32, Q4G };
-constexpr bool is_q4(WF f) { return f != WF::Q8; }
+// Weight formats: int8 codes (Q8Fine: sums as for int4, see tile_gemm_kernel), int4
+// codes with one scale per row, int4 in groups of 32 columns, int4 in groups of a
+// larger multiple of 32.
+enum class WF { Q8, Q8Fine, Q4Row, Q4G32, Q4G };
+constexpr bool is_q4(WF f) { return f != WF::Q8 && f != WF::Q8Fine; }
 constexpr bool is_grouped(WF f) { return f == WF::Q4G32 || f == WF::Q4G; }
 
 // n bytes at any address (global memory takes unaligned vector loads).
@@ -62,7 +64,10 @@ __device__ __forceinline__ int bf16_pair(float a, float b) {
 // significant bits, the next 8, the rest. An infinity keeps itself in the first
 // part and zeros in the others (inf - inf would be NaN). No branch here: the
 // conversions share a basic block with the MFMAs that they hide behind.
-__device__ __forceinline__ void split3(const float (&v)[8], v4i& hi, v4i& mid, v4i& lo) {
+// FINE: `lost` collects the bits that the parts drop, those of a smaller |v| and of a NaN
+// that has bits in its low half only.
+template <bool FINE>
+__device__ __forceinline__ void split3(const float (&v)[8], v4i& hi, v4i& mid, v4i& lo, unsigned& lost) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         float m[2], l[2];
@@ -70,9 +75,10 @@ __device__ __forceinline__ void split3(const float (&v)[8], v4i& hi, v4i& mid, v
         for (int e = 0; e < 2; ++e) {
             const float f = v[2 * i + e];
             float r = f - top16(f);
-            r = r == r ? r : 0.0f;
+            r = r == r ? r : FINE ? __builtin_bit_cast(float, bits(f) & 0xFFFFu) : 0.0f;
             m[e] = r;
             l[e] = r - top16(r);
+            if constexpr (FINE) lost |= bits(l[e]) & 0xFFFFu;
         }
         hi[i] = bf16_pair(v[2 * i], v[2 * i + 1]);
         mid[i] = bf16_pair(m[0], m[1]);
@@ -146,9 +152,10 @@ struct XPiece<float> {
             v[e] = c + e < k ? f : 0.0f;
         }
     }
-    __device__ __forceinline__ void store(int8_t* dst, int plane) const {
+    template <bool FINE>
+    __device__ __forceinline__ void store(int8_t* dst, int plane, unsigned& lost) const {
         v4i h, m, l;
-        split3(v, h, m, l);
+        split3<FINE>(v, h, m, l, lost);
         *reinterpret_cast<v4i*>(dst) = h;
         *reinterpret_cast<v4i*>(dst + plane) = m;
         *reinterpret_cast<v4i*>(dst + 2 * plane) = l;
@@ -168,7 +175,8 @@ struct XPiece<_Float16> {
         }
         v = __builtin_bit_cast(v4i, t);
     }
-    __device__ __forceinline__ void store(int8_t* dst, int) const { *reinterpret_cast<v4i*>(dst) = v; }
+    template <bool>
+    __device__ __forceinline__ void store(int8_t* dst, int, unsigned&) const { *reinterpret_cast<v4i*>(dst) = v; }
 };
 template <>
 struct XPiece<int8_t> {
@@ -188,7 +196,8 @@ struct XPiece<int8_t> {
             v[d] = static_cast<int>(u);
         }
     }
-    __device__ __forceinline__ void store(int8_t* dst, int) const { *reinterpret_cast<v4i*>(dst) = v; }
+    template <bool>
+    __device__ __forceinline__ void store(int8_t* dst, int, unsigned&) const { *reinterpret_cast<v4i*>(dst) = v; }
 };
 
 // PC (8 or 16) weight columns of one row. Columns past k keep whatever code the
@@ -252,13 +261,22 @@ struct TileArgs {
     int scale_f16, y_kind;      // y_kind: 0 fp32, 1 fp16, 2 int32 accumulators
 };
 
+__device__ __forceinline__ int chunk_group(const TileArgs& a, int chunk) {
+    return a.cpg == 1 ? chunk : static_cast<int>(__umulhi(static_cast<unsigned>(chunk), a.cpg_magic));
+}
+__device__ __forceinline__ float tile_scale(const TileArgs& a, size_t i) {
+    return a.scale_f16 ? static_cast<float>(static_cast<const _Float16*>(a.scale)[i]) : static_cast<const float*>(a.scale)[i];
+}
+
 template <typename XT, WF F, int WM, int WN, int FM, int FN, int SK>
 __global__ __launch_bounds__((WM * WN * 64)) void tile_gemm_kernel(TileArgs a) {
     using S = TileShape<XT, F, WM, WN, FM, FN, SK>;
     using XP = XPiece<XT>;
     constexpr bool I8 = sizeof(XT) == 1, BF = sizeof(XT) == 4, Q4 = is_q4(F), GROUPED = is_grouped(F);
     constexpr int NT = S::kThreads, T = S::kT, C = S::kC;
+    constexpr bool FINE = F != WF::Q8;  // never for int8 activations, whose sums are exact
     using Acc = std::conditional_t<I8, v4i, f4>;
+    using Sum = std::conditional_t<FINE, d4, Acc>;
     extern __shared__ __attribute__((aligned(16))) int8_t tile_lds[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -299,11 +317,8 @@ __global__ __launch_bounds__((WM * WN * 64)) void tile_gemm_kernel(TileArgs a) {
             for (int u = 0; u < S::kNS; ++u) {
                 const int i = tid + u * NT, row = min(n0 + i % S::kBN, n - 1);
                 const int chunk = slab * T + min(i / S::kBN, T - 1);  // int4 slabs: one chunk per MFMA step
-                int g = F == WF::Q4G32 ? chunk : static_cast<int>(__umulhi(static_cast<unsigned>(chunk), a.cpg_magic));
-                g = min(g, a.groups - 1);
-                const size_t o = static_cast<size_t>(row) * a.groups + g;
-                st.s[u] = a.scale_f16 ? static_cast<float>(static_cast<const _Float16*>(a.scale)[o])
-                                      : static_cast<const float*>(a.scale)[o];
+                const int g = min(chunk_group(a, chunk), a.groups - 1);
+                st.s[u] = tile_scale(a, static_cast<size_t>(row) * a.groups + g);
             }
         }
     };
@@ -322,11 +337,12 @@ __global__ __launch_bounds__((WM * WN * 64)) void tile_gemm_kernel(TileArgs a) {
         for (int u = 0; u < S::kNW; ++u) st.w[u].load_tail(wr[u], whole * SK + (tid + u * NT) % S::kWCpr * S::kPC, rb);
         load_scales(whole, st);
     };
+    unsigned lost[S::kNX] = {};
     auto store = [&](const Stage& st, int8_t* buf) {
 #pragma unroll
         for (int u = 0; u < S::kNX; ++u) {
             const int i = tid + u * NT, r = i / S::kXCpr, c = i % S::kXCpr;
-            if (S::kXU % NT == 0 || i < S::kXU) st.x[u].store(buf + r * S::kRow + ((c ^ tile_swz<C>(r)) << 4), S::kPlane);
+            if (S::kXU % NT == 0 || i < S::kXU) st.x[u].template store<FINE>(buf + r * S::kRow + ((c ^ tile_swz<C>(r)) << 4), S::kPlane, lost[u]);
         }
 #pragma unroll
         for (int u = 0; u < S::kNW; ++u) {
@@ -354,32 +370,37 @@ __global__ __launch_bounds__((WM * WN * 64)) void tile_gemm_kernel(TileArgs a) {
     };
 
     // Sums in two levels, as one chain over all of K rounds its running sum once per MFMA:
-    // fp32 activations start each chunk's three products from zero, largest part
-    // first, and `part` holds the sums of 256 columns or of the open group. (Smallest
-    // first is as good on one linear but leaves a mean error: the MFMA cuts the low
-    // bits of the sum it is given when larger products join, always downwards, m = 384,
-    // n = 896, k = 4864 -7.7e-8 of the rms against -1e-9, and a decoder's attention
-    // averages over such a shift without shrinking it: 2 layers, 384 tokens, int4 logits
-    // 6.5e-7 off and not 3.6e-7. Adding the largest part's product separately costs 5%.)
-    // The larger fp32 tiles on row scales add each chunk to the sum itself: `part` costs them
-    // the second workgroup of a CU (m = 333, n = 1536, k = 8960 47 -> 54 us). Relative
-    // errors against 64 bits, K whole, one chain -> this: Q8 fp32 k = 896 2.9e-7 ->
-    // 1.0e-7, fp16 k = 8960 5.7e-7 -> 1.4e-7; Q4G fp16 k = 4096 2.0e-7 -> 0.8e-7.
-    constexpr bool PART = !I8 && (!BF || GROUPED || FN * FM <= 4);
-    // Q4G closes a part with its group's scale; the others add it as it is.
-    constexpr bool GSCALE = F == WF::Q4G;
-    Acc acc[FN][FM];
+    // `part` holds the sums of 256 columns, and fp32 activations start each chunk's three
+    // products from zero, largest part first. (Smallest first is as good on one linear
+    // but leaves a mean error: the MFMA cuts the low bits of the sum it is given when
+    // larger products join, always downwards, m = 384, n = 896, k = 4864 -7.7e-8 of the rms
+    // against -1e-9, and a decoder's attention averages over such a shift without
+    // shrinking it: 2 layers, 384 tokens, int4 logits 6.5e-7 off and not 3.6e-7. Adding
+    // the largest part's product separately costs 5%.)
+    // Q8 on 16-byte rows of whole chunks stands for kernels of one chain: its larger
+    // fp32 tiles add each chunk to the sum itself, as `part` costs them the second
+    // workgroup of a CU (m = 333, n = 1536, k = 8960 47 -> 54 us).
+    // FINE, all others, stands for kernels that summed K in 64 lanes and a tree: it adds
+    // the parts in fp64 and sums again in fp64 what three bf16 parts cannot hold. Errors
+    // against 64 bits, those kernels / fp32 sums of the parts / this: one int4 group per
+    // row, fp32, m = 333, n = 9000, k = 8960 1.1e-7 / 2.3e-7 / 0.9e-7; groups of 64, fp16, k =
+    // 9000 7.5e-8 / 15e-8 / 6e-8; int8, fp32, k = 1003 1.02e-7 / 1.30e-7 / 0.94e-7. us, fp32
+    // sums -> this: int4 fp32, m = 333, n = 1536, k = 8960 groups of 32 61 -> 66, one group
+    // 51 -> 63; m = 1500, n = 6768, k = 2160 int8 fp32 182 -> 216, fp16 98 -> 102.
+    constexpr bool PART = !I8 && (FINE || !BF || FN * FM <= 4);
+    constexpr int kPart = FINE && !BF && !GROUPED ? 128 : 256;  // columns of a part
+    Sum acc[FN][FM];
     Acc part[PART ? FN : 1][PART ? FM : 1];
 #pragma unroll
     for (int i = 0; i < FN; ++i)
 #pragma unroll
         for (int j = 0; j < FM; ++j) {
-            acc[i][j] = Acc{0, 0, 0, 0};
+            acc[i][j] = Sum{0, 0, 0, 0};
             if constexpr (PART) part[i][j] = Acc{0, 0, 0, 0};
         }
     const int xrow = wm * FM * 16 + fr, wrow = wn * FN * 16 + fr;
     const int xsw = tile_swz<C>(xrow), wsw = tile_swz<C>(wrow);  // a 16-row step keeps the swizzle
-    // The MFMAs of a slab in LDS; flush(t): whether step t closes a group or a part.
+    // The MFMAs of a slab in LDS; flush(t): whether step t closes a part.
     auto compute = [&](const int8_t* buf, auto flush) {
 #pragma unroll
         for (int t = 0; t < T; ++t) {
@@ -418,9 +439,8 @@ __global__ __launch_bounds__((WM * WN * 64)) void tile_gemm_kernel(TileArgs a) {
                                                                        __builtin_bit_cast(h8, wb[i]), d, 0, 0, 0);
                         }
                         if constexpr (F == WF::Q4G32) {
-                            Acc& to = PART ? part[PART ? i : 0][PART ? j : 0] : acc[i][j];
 #pragma unroll
-                            for (int v = 0; v < 4; ++v) to[v] = __builtin_fmaf(d[v], sc[i], to[v]);
+                            for (int v = 0; v < 4; ++v) part[i][j][v] = __builtin_fmaf(d[v], sc[i], part[i][j][v]);
                         } else if constexpr (PART && BF) {
 #pragma unroll
                             for (int v = 0; v < 4; ++v) part[i][j][v] += d[v];
@@ -442,9 +462,13 @@ __global__ __launch_bounds__((WM * WN * 64)) void tile_gemm_kernel(TileArgs a) {
 #pragma unroll
                         for (int j = 0; j < FM; ++j) {
 #pragma unroll
-                            for (int v = 0; v < 4; ++v)
-                                acc[i][j][v] = GSCALE ? __builtin_fmaf(part[i][j][v], sc[GSCALE ? i : 0], acc[i][j][v])
-                                                      : acc[i][j][v] + part[i][j][v];
+                            for (int v = 0; v < 4; ++v) {
+                                // Q4G closes a part with its group's scale; the others add it as it is.
+                                if constexpr (F == WF::Q4G)
+                                    acc[i][j][v] = __builtin_fma(static_cast<double>(part[i][j][v]), static_cast<double>(sc[i]), acc[i][j][v]);
+                                else
+                                    acc[i][j][v] += part[i][j][v];
+                            }
                             part[i][j] = Acc{0, 0, 0, 0};
                         }
                 }
@@ -471,15 +495,15 @@ __global__ __launch_bounds__((WM * WN * 64)) void tile_gemm_kernel(TileArgs a) {
         auto body = [&](int i, Stage& a0, Stage& a1) {  // a0 free, a1 = slab i + 1
             load(min(first + i + 2, s1 - 1), a0);
             __builtin_amdgcn_sched_barrier(0);  // the loads stay two slabs ahead: left alone they sank to the barrier
-            const bool is_tail = tail && i == 0, last = i == nk - 1;
+            const bool is_tail = tail && i == 0, full = i == nk - 1 || i % (kPart / SK) == 0;
             compute(cur, [&](int t) {
                 if constexpr (F == WF::Q4G) {
                     if (is_tail) return true;
                     const bool end_of_group = ++pos == a.cpg;
                     if (end_of_group) pos = 0;
-                    return end_of_group || (last && t == T - 1);
+                    return end_of_group || (full && t == T - 1);
                 } else {
-                    return t == T - 1 && (last || i % (256 / SK) == 0);
+                    return full && t == T - 1;
                 }
             });
             store(a1, nxt);  // past the last slab: a repeat nobody reads
@@ -512,44 +536,104 @@ __global__ __launch_bounds__((WM * WN * 64)) void tile_gemm_kernel(TileArgs a) {
         compute(tile_lds, [&](int) { return true; });
     }
 
-    // Lane l holds, of fragment (i, j), rows 4 * (l / 16) + v of column l % 16.
     const size_t plane = static_cast<size_t>(blockIdx.y) * m * n;
+    auto put = [&](int row, int col, float ws, float b, auto sum) {
+        const size_t o = static_cast<size_t>(row) * n + col;
+        float r;
+        if constexpr (I8) {
+            if (a.planes) {
+                static_cast<int32_t*>(a.planes)[plane + o] = sum;
+                return;
+            }
+            if (a.y_kind == 2) {
+                static_cast<int32_t*>(a.y)[o] = sum;
+                return;
+            }
+            r = w8a8_epilogue(sum, a.a_scale[row], ws, b);
+        } else {
+            if (a.planes) {
+                static_cast<float*>(a.planes)[plane + o] = static_cast<float>(sum);
+                return;
+            }
+            r = static_cast<float>(GROUPED ? sum + b : sum * ws + b);
+        }
+        if (a.y_kind == 1) static_cast<_Float16*>(a.y)[o] = from_f32<_Float16>(r);
+        else static_cast<float*>(a.y)[o] = r;
+    };
+    const bool scaled = !a.planes && a.y_kind != 2;
+
+    // FINE fp32: an output of a row that dropped bits (less than 2^-133 of each value, so
+    // 2^-126 of each product with a code) is summed again in fp64 where these are over
+    // 2^-27 of it, that is where the whole row is tiny, or where it is no number.
+    unsigned* redo = reinterpret_cast<unsigned*>(tile_lds);  // a bit per output of the tile
+    __shared__ unsigned lost_rows[(S::kBM + 31) / 32];
+    unsigned any_lost = 0;
+    double least[FN] = {};
+    if constexpr (FINE && BF) {
+        constexpr int words = (S::kBM + 31) / 32;
+        if (tid < words) lost_rows[tid] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < S::kNX; ++u) {
+            const int r = (tid + u * NT) / S::kXCpr;
+            if (lost[u]) atomicOr(&lost_rows[r >> 5], 1u << (r & 31));
+        }
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < words; ++i) any_lost |= lost_rows[i];
+        if (any_lost) {
+            for (int i = tid; i < S::kBM * S::kBN / 32; i += NT) redo[i] = 0;
+#pragma unroll
+            for (int i = 0; i < FN; ++i) {
+                float top = GROUPED ? 0.0f : 1.0f;
+                if constexpr (GROUPED)
+                    for (int g = 0; g < a.groups; ++g)
+                        top = fmaxf(top, fabsf(tile_scale(a, static_cast<size_t>(min(n0 + wrow + i * 16, n - 1)) * a.groups + g)));
+                least[i] = 0x1p-99 * (nk * SK) * top;
+            }
+            __syncthreads();
+        }
+    }
+    // Lane l holds, of fragment (i, j), rows 4 * (l / 16) + v of column l % 16.
 #pragma unroll
     for (int i = 0; i < FN; ++i) {
         const int col = n0 + wrow + i * 16;
         if (col >= n) continue;
-        float ws = 1.0f, b = 0.0f;
-        if (!a.planes && a.y_kind != 2) {
-            if constexpr (!GROUPED)
-                ws = a.scale_f16 ? static_cast<float>(static_cast<const _Float16*>(a.scale)[col])
-                                 : static_cast<const float*>(a.scale)[col];
-            if (a.bias) b = a.bias[col];
-        }
+        const float ws = scaled && !GROUPED ? tile_scale(a, col) : 1.0f, b = scaled && a.bias ? a.bias[col] : 0.0f;
 #pragma unroll
         for (int j = 0; j < FM; ++j)
 #pragma unroll
             for (int v = 0; v < 4; ++v) {
-                const int row = m0 + wm * FM * 16 + j * 16 + 4 * fq + v;
-                if (row >= m) continue;
-                const size_t o = static_cast<size_t>(row) * n + col;
-                if constexpr (I8) {
-                    if (a.planes) static_cast<int32_t*>(a.planes)[plane + o] = acc[i][j][v];
-                    else if (a.y_kind == 2) static_cast<int32_t*>(a.y)[o] = acc[i][j][v];
-                    else {
-                        const float r = w8a8_epilogue(acc[i][j][v], a.a_scale[row], ws, b);
-                        if (a.y_kind == 1) static_cast<_Float16*>(a.y)[o] = from_f32<_Float16>(r);
-                        else static_cast<float*>(a.y)[o] = r;
-                    }
-                } else {
-                    if (a.planes) {
-                        static_cast<float*>(a.planes)[plane + o] = acc[i][j][v];
+                const int r = wm * FM * 16 + j * 16 + 4 * fq + v;
+                if (m0 + r >= m) continue;
+                if constexpr (FINE && BF) {
+                    const double t = fabs(acc[i][j][v]);
+                    if (any_lost && (lost_rows[r >> 5] >> (r & 31) & 1) && !(t >= least[i] && t < __builtin_inf())) {
+                        const int e = r * S::kBN + col - n0;
+                        atomicOr(&redo[e >> 5], 1u << (e & 31));
                         continue;
                     }
-                    const float r = GROUPED ? acc[i][j][v] + b : acc[i][j][v] * ws + b;
-                    if (a.y_kind == 1) static_cast<_Float16*>(a.y)[o] = from_f32<_Float16>(r);
-                    else static_cast<float*>(a.y)[o] = r;
                 }
+                put(m0 + r, col, ws, b, acc[i][j][v]);
             }
+    }
+    if constexpr (FINE && BF) {
+        if (!any_lost) return;
+        __syncthreads();
+        for (int e = tid; e < S::kBM * S::kBN; e += NT) {
+            if (!(redo[e >> 5] >> (e & 31) & 1)) continue;
+            const int row = m0 + e / S::kBN, col = n0 + e % S::kBN;
+            const XT* xp = static_cast<const XT*>(a.x) + static_cast<size_t>(row) * k;
+            const uint8_t* wp = a.w + static_cast<size_t>(col) * rb;
+            double sum = 0.0;
+            for (int c = s0 * SK; c < min(k, end * SK); ++c) {
+                const int q = Q4 ? ((wp[c >> 1] >> (4 * (c & 1))) & 15) - 8 : static_cast<int8_t>(wp[c]);
+                double t = static_cast<double>(xp[c]) * q;
+                if constexpr (GROUPED) t *= tile_scale(a, static_cast<size_t>(col) * a.groups + chunk_group(a, c >> 5));
+                sum += t;
+            }
+            put(row, col, scaled && !GROUPED ? tile_scale(a, col) : 1.0f, scaled && a.bias ? a.bias[col] : 0.0f, sum);
+        }
     }
 }
 
@@ -566,7 +650,7 @@ __global__ __launch_bounds__(256) void tile_reduce_kernel(TileArgs a, int splits
 #pragma unroll
     for (int sp = 0; sp < kTileMaxSplits; ++sp)
         if (sp < splits) v[sp] = part[sp * mn + i];
-    V t = v[0];
+    std::conditional_t<I8, int32_t, double> t = v[0];
 #pragma unroll
     for (int sp = 1; sp < kTileMaxSplits; ++sp)
         if (sp < splits) t += v[sp];
@@ -577,14 +661,11 @@ __global__ __launch_bounds__(256) void tile_reduce_kernel(TileArgs a, int splits
         }
     }
     const int col = static_cast<int>(i % a.n);
-    float ws = 1.0f;
-    if (row_scale)
-        ws = a.scale_f16 ? static_cast<float>(static_cast<const _Float16*>(a.scale)[col])
-                         : static_cast<const float*>(a.scale)[col];
+    const float ws = row_scale ? tile_scale(a, col) : 1.0f;
     const float b = a.bias ? a.bias[col] : 0.0f;
     float r;
     if constexpr (I8) r = w8a8_epilogue(t, a.a_scale[i / a.n], ws, b);
-    else r = t * ws + b;
+    else r = static_cast<float>(t * ws + b);
     if (a.y_kind == 1) static_cast<_Float16*>(a.y)[i] = from_f32<_Float16>(r);
     else static_cast<float*>(a.y)[i] = r;
 }
@@ -609,7 +690,7 @@ struct TileDim {
 constexpr int kTileCount = 5;
 constexpr TileDim kTiles[kTileCount] = {{128, 128}, {64, 128}, {64, 64}, {32, 64}, {16, 64}};
 constexpr TileModel kTileModels[] = {
-    // fp32 activations; the same with int4 groups; fp16; with int4 groups; int8
+    // fp32 activations; the same with fine sums; fp16; with fine sums; int8
     {4.5f, 1.1f, 2.9f, {{3.1f, 0.898f, 0.657f}, {3.5f, 0.7f, 0.422f}, {2.8f, 0.462f, 0.288f}, {1.1f, 0.476f, 0.209f}, {0.4f, 0.362f, 0.164f}}},
     {4.5f, 1.2f, 2.8f, {{3.1f, 0.982f, 0.921f}, {3.3f, 0.756f, 0.477f}, {2.4f, 0.513f, 0.322f}, {1.f, 0.463f, 0.269f}, {0.f, 0.397f, 0.243f}}},
     {4.1f, 1.4f, 4.f, {{7.7f, 0.843f, 0.574f}, {6.2f, 0.576f, 0.371f}, {5.f, 0.364f, 0.234f}, {2.7f, 0.252f, 0.17f}, {1.1f, 0.258f, 0.162f}}},
@@ -622,8 +703,8 @@ struct TilePlan {
     int cfg, splits;
     double us;  // modelled time
 };
-TilePlan plan_tile(TileX xt, bool grouped, int64_t m, int64_t n, int64_t k, int64_t ws_bytes) {
-    const TileModel& mod = kTileModels[xt == TileX::I8 ? 4 : (xt == TileX::F16 ? 2 : 0) + (grouped ? 1 : 0)];
+TilePlan plan_tile(TileX xt, bool fine, int64_t m, int64_t n, int64_t k, int64_t ws_bytes) {
+    const TileModel& mod = kTileModels[xt == TileX::I8 ? 4 : (xt == TileX::F16 ? 2 : 0) + (fine ? 1 : 0)];
     const int64_t sk = xt == TileX::F32 ? 32 : xt == TileX::F16 ? 64 : 128, slabs = (k + sk - 1) / sk;
     const double mn = static_cast<double>(m) * n;
     TilePlan best{kTileCount - 1, 1, 0};
@@ -675,9 +756,9 @@ template <typename XT, WF F>
 nq_status launch_tile_cfg(const TileArgs& a, int cfg, int splits, hipStream_t s) {
     switch (cfg) {
         case 0:
-            // fp32 activations: eight waves, as three planes of fragments per wave of
-            // four leave too few registers
-            if constexpr (sizeof(XT) == 4) return launch_tile<XT, F, 4, 2, 2, 4>(a, splits, s);
+            // fp32 activations and fp64 sums: eight waves, as three planes of fragments (the
+            // sums) per wave of four leave too few registers
+            if constexpr (sizeof(XT) == 4 || F != WF::Q8) return launch_tile<XT, F, 4, 2, 2, 4>(a, splits, s);
             else return launch_tile<XT, F, 2, 2, 4, 4>(a, splits, s);
         case 1: return launch_tile<XT, F, 2, 2, 2, 4>(a, splits, s);
         case 2: return launch_tile<XT, F, 2, 2, 2, 2>(a, splits, s);
@@ -690,8 +771,9 @@ template <typename XT>
 nq_status launch_tile_fmt(const TileArgs& a, WF f, int cfg, int splits, hipStream_t s) {
     switch (f) {
         case WF::Q8: return launch_tile_cfg<XT, WF::Q8>(a, cfg, splits, s);
-        case WF::Q4Row: return launch_tile_cfg<XT, WF::Q4Row>(a, cfg, splits, s);
         case WF::Q4G32: return launch_tile_cfg<XT, WF::Q4G32>(a, cfg, splits, s);
+        case WF::Q8Fine: return launch_tile_cfg<XT, WF::Q8Fine>(a, cfg, splits, s);
+        case WF::Q4Row: return launch_tile_cfg<XT, WF::Q4Row>(a, cfg, splits, s);
         default: return launch_tile_cfg<XT, WF::Q4G>(a, cfg, splits, s);
     }
 }
@@ -704,19 +786,19 @@ bool tile_gemm_ok(bool q4, int64_t m, int64_t n, int64_t k, int64_t group) {
     return ((m + 15) / 16) * ((n + 63) / 64) <= (int64_t(1) << 24);  // tiles, and chunks * cpg, in 32 bits
 }
 
-size_t tile_gemm_ws_bytes(TileX xt, bool grouped, int64_t m, int64_t n, int64_t k) {
-    const TilePlan p = plan_tile(xt, grouped, m, n, k, kTilePlanesMax);
+size_t tile_gemm_ws_bytes(TileX xt, bool fine, int64_t m, int64_t n, int64_t k) {
+    const TilePlan p = plan_tile(xt, fine, m, n, k, kTilePlanesMax);
     return p.splits > 1 ? round_up(static_cast<size_t>(p.splits) * m * n * 4, 256) : 0;
 }
 
-bool tile_gemm_split_fits(TileX xt, bool grouped, int64_t m, int64_t n, int64_t k, size_t ws_bytes) {
+bool tile_gemm_split_fits(TileX xt, bool fine, int64_t m, int64_t n, int64_t k, size_t ws_bytes) {
     const int64_t have = static_cast<int64_t>(std::min<size_t>(ws_bytes, kTilePlanesMax));
-    return plan_tile(xt, grouped, m, n, k, have).us <= 1.25 * plan_tile(xt, grouped, m, n, k, kTilePlanesMax).us;
+    return plan_tile(xt, fine, m, n, k, have).us <= 1.25 * plan_tile(xt, fine, m, n, k, kTilePlanesMax).us;
 }
 
 nq_status tile_gemm(const TileCall& c, void* ws, size_t ws_bytes, hipStream_t s) {
     const bool row = c.q4 && c.group >= c.k, grouped = c.q4 && !row;
-    const TilePlan p = plan_tile(c.xt, grouped, c.m, c.n, c.k, ws ? static_cast<int64_t>(std::min<size_t>(ws_bytes, kTilePlanesMax)) : 0);
+    const TilePlan p = plan_tile(c.xt, c.q4 || c.fine, c.m, c.n, c.k, ws ? static_cast<int64_t>(std::min<size_t>(ws_bytes, kTilePlanesMax)) : 0);
     TileArgs a{};
     a.x = c.x;
     a.w = c.w;
@@ -733,7 +815,7 @@ nq_status tile_gemm(const TileCall& c, void* ws, size_t ws_bytes, hipStream_t s)
     a.cpg = grouped ? static_cast<int>(c.group / 32) : 1;
     a.groups = grouped ? static_cast<int>((c.k + c.group - 1) / c.group) : 1;
     a.cpg_magic = a.cpg > 1 ? static_cast<unsigned>(((uint64_t(1) << 32) + a.cpg - 1) / a.cpg) : 0;
-    const WF f = !c.q4 ? WF::Q8 : row ? WF::Q4Row : c.group == 32 ? WF::Q4G32 : WF::Q4G;
+    const WF f = !c.q4 ? c.fine ? WF::Q8Fine : WF::Q8 : row ? WF::Q4Row : c.group == 32 ? WF::Q4G32 : WF::Q4G;
     if (c.xt == TileX::F32) return launch_tile_fmt<float>(a, f, p.cfg, p.splits, s);
     if (c.xt == TileX::F16) return launch_tile_fmt<_Float16>(a, f, p.cfg, p.splits, s);
     return launch_tile_cfg<int8_t, WF::Q8>(a, p.cfg, p.splits, s);

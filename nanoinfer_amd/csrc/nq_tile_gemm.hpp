@@ -21,15 +21,16 @@ struct TileCall {
     void* y;
     TileY yt;
     int64_t m, n, k;
+    bool fine;  // int8 codes, F32 / F16: sums no coarser than 64 lanes and a tree (int4: always)
 };
 
 // Whether the tile GEMM takes these operands: any pointer alignment, any k up to 2^20.
 bool tile_gemm_ok(bool q4, int64_t m, int64_t n, int64_t k, int64_t group);
 // Workspace its split-K planes take at this shape (0: no split); less or none is accepted
-// and splits less.
-size_t tile_gemm_ws_bytes(TileX xt, bool grouped, int64_t m, int64_t n, int64_t k);
+// and splits less. fine: int4 codes, or TileCall::fine.
+size_t tile_gemm_ws_bytes(TileX xt, bool fine, int64_t m, int64_t n, int64_t k);
 // Whether the plan within ws_bytes comes within a quarter of the unlimited one.
-bool tile_gemm_split_fits(TileX xt, bool grouped, int64_t m, int64_t n, int64_t k, size_t ws_bytes);
+bool tile_gemm_split_fits(TileX xt, bool fine, int64_t m, int64_t n, int64_t k, size_t ws_bytes);
 nq_status tile_gemm(const TileCall& c, void* ws, size_t ws_bytes, hipStream_t s);
 
 // The same operands at m <= 8 (nq_gemv_any.hip); no workspace.

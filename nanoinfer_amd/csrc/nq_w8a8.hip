@@ -830,7 +830,7 @@ nq_status run_gemm(const int8_t* xq, const float* as, const int8_t* wq, const fl
                    int64_t n, int64_t k, void* workspace, size_t ws_bytes, int path, hipStream_t s) {
     int p = resolve_path(path, m, n, k);
     const TileCall tile{TileX::I8, xq, reinterpret_cast<const uint8_t*>(wq), false, ws, false, 0, as, bias,
-                        acc_out ? acc_out : y, acc_out ? kTileI32 : ydt == NQ_F32 ? kTileF32 : kTileF16, m, n, k};
+                        acc_out ? acc_out : y, acc_out ? kTileI32 : ydt == NQ_F32 ? kTileF32 : kTileF16, m, n, k, false};
     if (path == NQ_PATH_AUTO && m <= 8 && !mfma_ok(xq, wq, k) && tile_gemm_ok(false, m, n, k, 0)) return gemv_any(tile, s);
     if (path == NQ_PATH_AUTO && w8a8_tile_route(mfma_ok(xq, wq, k), m, n, k)) return tile_gemm(tile, workspace, ws_bytes, s);
     if (p == NQ_PATH_MFMA && !mfma_ok(xq, wq, k)) p = NQ_PATH_GENERIC;

@@ -1206,7 +1206,7 @@ bool wq_tile_route(bool q4, bool f32x, bool scale_f16, bool general, bool slices
         const WqRoute r = plan_wq_route(m, n, k, !few, true, sk64, false, ws, q4);
         take = !r.wide || (m >= 65 && (r.splits > 1 || m * n <= (int64_t(3) << 19)));
     }
-    return take && (ws || tile_gemm_split_fits(f32x ? TileX::F32 : TileX::F16, q4 && !row, m, n, k, 0));
+    return take && (ws || tile_gemm_split_fits(f32x ? TileX::F32 : TileX::F16, q4, m, n, k, 0));
 }
 
 // The split-K planes that the tile GEMM uses when the workspace holds them, for any
@@ -1215,7 +1215,7 @@ size_t wq_tile_ws_bytes(int64_t m, int64_t n, int64_t k) {
     if (m < 9 || (m < 16 && k % 32 == 0) || !tile_gemm_ok(false, m, n, k, 0)) return 0;
     size_t most = 0;
     for (TileX xt : {TileX::F32, TileX::F16})
-        for (bool grouped : {false, true}) most = std::max(most, tile_gemm_ws_bytes(xt, grouped, m, n, k));
+        for (bool fine : {false, true}) most = std::max(most, tile_gemm_ws_bytes(xt, fine, m, n, k));
     return most;
 }
 

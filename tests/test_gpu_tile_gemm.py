@@ -38,7 +38,7 @@ def _check(y, x, wd, b, k):
         lim = lim + 2.0 ** -10 * ref.abs() + 2.0 ** -24
     assert y.shape == ref.shape
     assert bool(((y.double() - ref).abs() <= lim).all())
-    if y.dtype == F32:  # the bound is loose by sqrt(k): measured 1e-7 on all plans
+    if y.dtype == F32:  # the bound is loose by sqrt(k); test_errors_on_long_k has the tight one
         assert float((y.double() - ref).norm() / ref.norm()) < 2e-6
 
 
@@ -95,6 +95,53 @@ def test_gemv(dev, nq, xdt, fmt, group):
         b = torch.randn(n, generator=g, device=dev) if i % 3 else None
         y = (nq.linear_q8 if fmt == "q8" else nq.linear_q4g)(x, t, b, F16 if i % 4 == 3 else F32)
         _check(y, x, _codes(t, gr), b, k)
+
+
+# int8 on aligned rows of whole chunks, whose larger tiles add their sums in fp32
+@gpu
+@pytest.mark.parametrize("xdt", [F32, F16])
+@pytest.mark.parametrize("m,n,k", [(1000, 4001, 1056), (1300, 5001, 1056)])
+def test_q8_of_whole_chunks(dev, nq, xdt, m, n, k):
+    g = torch.Generator(device=dev).manual_seed(n)
+    t, _ = _make(nq, "q8", n, k, 0, F32, g)
+    x, b = torch.randn(m, k, generator=g, device=dev).to(xdt), torch.randn(n, generator=g, device=dev)
+    for ydt in (F32, F16):
+        _check(nq.linear_q8(x, t, b, ydt), x, _codes(t, 0), b, k)
+
+
+# Errors against 64 bits on long and odd K. The kernels before these summed K in 64 lanes
+# and a tree; a result here rounds its sums over 256 columns (at most 8 additions that each
+# hold j / 8 of the sum, (1 + ... + 8) / 8 = 4.5 roundings in quadrature; fp16 groups and
+# int8 half as many), a plane (1), the end (1) and, for fp32 x, the three parts' MFMAs of a
+# chunk (at most 3), each 2^-24 / sqrt(3) at most: sqrt(9.5) and sqrt(6.5) of these.
+@gpu
+@pytest.mark.parametrize("xdt", [F32, F16])
+@pytest.mark.parametrize("fmt,group", [("q8", 0), ("q4", 0), ("q4g", 32), ("q4g", 64), ("q4g", 96), ("q4g", 256)])
+def test_errors_on_long_k(dev, nq, xdt, fmt, group):
+    g = torch.Generator(device=dev).manual_seed(group)
+    lim = 2.0 ** -24 * ((9.5 if xdt == F32 else 6.5) / 3) ** 0.5
+    for m, n, k in ((4, 200, 8955), (8, 2100, 1003), (12, 256, 1003), (130, 515, 8955),
+                    (333, 4500, 8960 if fmt == "q4" else 9001), (600, 4001, 1003)):
+        t, gr = _make(nq, fmt, n, k, group, F32, g)
+        x = torch.randn(m, k, generator=g, device=dev).to(xdt)
+        # odd rows: fp32 values whose three bf16 parts drop bits; fp16 subnormals
+        x[1::2] *= 2.0 ** -116 if xdt == F32 else 2.0 ** -18
+        ref = x.double() @ _codes(t, gr).t().contiguous()
+        d = (nq.linear_q8 if fmt == "q8" else nq.linear_q4g)(x, t, None, F32).double() - ref
+        for rows in (slice(0, None, 2), slice(1, None, 2)):
+            assert float(d[rows].norm() / ref[rows].norm()) < lim, (m, n, k, rows)
+
+
+@gpu
+def test_nan_with_low_bits_only(dev, nq):
+    """A NaN whose upper half reads as an infinity stays a NaN in every output of its row."""
+    for m, k in ((3, 259), (40, 259), (300, 1003)):
+        x = torch.randn(m, k, device=dev)
+        x.view(torch.int32)[1, 7] = 0x7F800001
+        for t, f in ((nq.quantize_q8(torch.randn(200, k, device=dev)), nq.linear_q8),
+                     (nq.quantize_q4g(torch.randn(200, k, device=dev), 32), nq.linear_q4g)):
+            y = f(x, t)
+            assert bool(torch.isnan(y[1]).all()) and bool(torch.isfinite(y[0]).all()) and bool(torch.isfinite(y[2:]).all())
 
 
 # fp32 rows: the errors have no common sign. The mean over 344064 outputs of errors of at
