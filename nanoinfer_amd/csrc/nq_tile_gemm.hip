@@ -384,7 +384,7 @@ __global__ __launch_bounds__((WM * WN * 64)) void tile_gemm_kernel(TileArgs a) {
     // the parts in fp64 and sums again in fp64 what three bf16 parts cannot hold. Errors
     // against 64 bits, those kernels / fp32 sums of the parts / this: one int4 group per
     // row, fp32, m = 333, n = 9000, k = 8960 1.1e-7 / 2.3e-7 / 0.9e-7; groups of 64, fp16, k =
-    // 9000 7.5e-8 / 15e-8 / 6e-8; int8, fp32, k = 1003 1.02e-7 / 1.30e-7 / 0.94e-7. us, fp32
+    // 9000 7.5e-8 / 15e-8 / 4e-8; int8, fp32, k = 1003 1.02e-7 / 1.30e-7 / 0.94e-7. us, fp32
     // sums -> this: int4 fp32, m = 333, n = 1536, k = 8960 groups of 32 61 -> 66, one group
     // 51 -> 63; m = 1500, n = 6768, k = 2160 int8 fp32 182 -> 216, fp16 98 -> 102.
     constexpr bool PART = !I8 && (FINE || !BF || FN * FM <= 4);

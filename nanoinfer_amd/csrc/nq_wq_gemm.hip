@@ -383,13 +383,6 @@ struct WqRowPlan {
     int tm, tn, splits, per;
 };
 
-// Split K of the 16-row kernel: up to 32 rows of x, and with fp32 x on weights of up to
-// 4096 rows from m = 17; the tile GEMM has the rest.
-template <typename XT>
-constexpr bool wq_row_split_built(int tm, int tn) {
-    return tm == 1 || (tm == 2 && (sizeof(XT) == 2 || tn == 1));
-}
-
 template <bool Q4, typename XT, typename YT, typename ST>
 nq_status launch_wq(const XT* x, const uint8_t* w, const ST* sc, const float* b, YT* y, int m, int n, int k,
                     int g, WqRowPlan p, float* planes, hipStream_t s) {
@@ -405,15 +398,12 @@ nq_status launch_wq(const XT* x, const uint8_t* w, const ST* sc, const float* b,
     auto go = [&](auto tmtag, auto tntag) {
         constexpr int TM = decltype(tmtag)::value, TN = decltype(tntag)::value;
         const dim3 grid(static_cast<unsigned>((n + 16 * TN - 1) / (16 * TN)), mblocks, static_cast<unsigned>(p.splits));
-        if constexpr (wq_row_split_built<XT>(TM, TN)) {
-            if (planes) {
-                gemm_wq_kernel<Q4, TM, TN, XT, YT, ST, true><<<grid, wq_waves<TM>() * 64, 0, s>>>(x, w, sc, b, y, m, n, k,
-                                                                                                 g, planes, p.per);
-                return;
-            }
-        }
-        gemm_wq_kernel<Q4, TM, TN, XT, YT, ST><<<grid, wq_waves<TM>() * 64, 0, s>>>(x, w, sc, b, y, m, n, k, g,
-                                                                                   nullptr, p.per);
+        if (planes)
+            gemm_wq_kernel<Q4, TM, TN, XT, YT, ST, true><<<grid, wq_waves<TM>() * 64, 0, s>>>(x, w, sc, b, y, m, n, k,
+                                                                                             g, planes, p.per);
+        else
+            gemm_wq_kernel<Q4, TM, TN, XT, YT, ST><<<grid, wq_waves<TM>() * 64, 0, s>>>(x, w, sc, b, y, m, n, k, g,
+                                                                                       nullptr, p.per);
     };
     auto with_tn = [&](auto tmtag) {
         if constexpr (decltype(tmtag)::value <= 2) {
@@ -818,7 +808,7 @@ nq_status launch_wq_wide(const XT* x, const uint8_t* w, const ST* sc, const floa
 // two 91.9, 256 x 128 in three 100).
 struct WqTile {
     int fm, fn, sk;
-    bool shallow = false;  // a two-slot ring (fm = 1, fn = 2): more workgroups per CU
+    bool shallow = false;  // a two-slot ring (fm = 1, fn = 2 or 4): more workgroups per CU
 };
 constexpr WqTile kWqTiles[] = {{4, 9, 64}, {4, 8, 64}, {2, 9, 128}, {4, 4, 64}, {2, 8, 128},
                                {2, 4, 128}, {1, 8, 128}, {1, 4, 128}, {1, 2, 128}};
@@ -888,7 +878,7 @@ nq_status wq_wide_tiles(const XT* x, const uint8_t* w, const ST* sc, const float
         constexpr int SK = decltype(skt)::value, FM = decltype(fmt)::value, FN2 = decltype(fnt)::value;
         constexpr int WN = Q4 ? 2 : FN2 % 3 == 0 ? 3 : FN2 % 4 == 0 ? 4 : 2, FN = FN2 * 2 / WN;
         using D8 = integral_constant<int, 8>;
-        if constexpr (!F32X && FM == 1 && FN2 == 2) {
+        if constexpr (FM == 1 && (FN2 == 2 || FN2 == 4)) {
             if (pick.shallow)  // two ring slots: two or three workgroups per CU
                 return launch_g(skt, fmt, integral_constant<int, FN>{}, integral_constant<int, WN>{},
                                 integral_constant<int, 4>{}, integral_constant<int, 2>{});
@@ -1057,12 +1047,6 @@ WqRoute plan_wq_route(int64_t m, int64_t n, int64_t k, bool wide_ok, bool wide_c
     r.per = p.per;
     return r;
 }
-// Whether a split route has its kernels here; the tile GEMM took the others over. Their
-// planes stay in the required workspace, whose size callers were given.
-template <typename XT>
-bool wq_split_built(const WqRoute& r) {
-    return r.wide ? sizeof(XT) == 2 && r.tile.fn == 2 : wq_row_split_built<XT>(r.row.tm, r.row.tn);
-}
 size_t wq_route_bytes(const WqRoute& r, int64_t m, int64_t n) {
     return r.splits > 1 ? round_up(static_cast<size_t>(r.splits) * static_cast<size_t>(m) * static_cast<size_t>(n) * 4, 256) : 0;
 }
@@ -1158,7 +1142,7 @@ nq_status wq_gemm(const XT* x, const uint8_t* w, const ST* sc, const float* b, Y
     const bool sk64 = wq_sk64_ok<Q4, ST>(group), f32x = sizeof(XT) == 4;
     const bool wide_ok = wq_wide_ok<Q4, XT, ST>(m, n, k, group), contract = wq_wide_contract<Q4, XT, ST>(m, n, k, group);
     WqRoute r = plan_wq_route(m, n, k, wide_ok, contract, sk64, f32x, workspace != nullptr, Q4);
-    if (r.splits > 1 && (!wq_split_built<XT>(r) || workspace_bytes < wq_route_bytes(r, m, n)))
+    if (r.splits > 1 && workspace_bytes < wq_route_bytes(r, m, n))
         r = plan_wq_route(m, n, k, wide_ok, contract, sk64, f32x, false, Q4);
     float* planes = r.splits > 1 ? static_cast<float*>(workspace) : nullptr;
     const int mi = static_cast<int>(m), ni = static_cast<int>(n), ki = static_cast<int>(k), gi = static_cast<int>(group);

@@ -211,6 +211,38 @@ def test_neighbours_of_the_route(dev, nq, xdt, m, n, k, fmt, sdt):
         _check((nq.linear_q8 if fmt == "q8" else nq.linear_q4g)(x, t, None, ydt), x, _codes(t, gr), None, k)
 
 
+def _call(lib, x, t, y, ws, nbytes, path):
+    """nq_linear_q8_ex / nq_linear_q4g_ex on a workspace of the caller."""
+    f = lambda d: 0 if d == F32 else 1
+    tail = (None, y.data_ptr(), f(y.dtype), x.shape[0], t.out, t.in_, ws.data_ptr() if nbytes else None, nbytes, path,
+            torch.cuda.current_stream().cuda_stream)
+    if hasattr(t, "group"):
+        return lib.nq_linear_q4g_ex(x.data_ptr(), f(x.dtype), t.q.data_ptr(), t.scale.data_ptr(), f(t.scale.dtype), t.group, *tail)
+    return lib.nq_linear_q8_ex(x.data_ptr(), f(x.dtype), t.q.data_ptr(), t.scale.data_ptr(), *tail)
+
+
+# The explicit MFMA path on the workspace that it requires splits K, as its planes there
+# show: 64-row tiles of 64 and 128 columns, 16-row tiles of 17 to 32, 33 to 48 and more rows.
+@gpu
+@pytest.mark.parametrize("xdt", [F32, F16])
+@pytest.mark.parametrize("m,n,k", [(40, 130, 2048), (100, 130, 2048), (24, 130, 4128), (24, 4200, 4128), (40, 130, 4128),
+                                   (100, 130, 4128)])
+def test_explicit_mfma_splits_k(dev, nq, xdt, m, n, k):
+    from nanoinfer_amd import _lib
+    lib, g = _lib.load(), torch.Generator(device=dev).manual_seed(m + n + k)
+    x = torch.randn(m, k, generator=g, device=dev).to(xdt)
+    need = lib.nq_linear_wq_workspace_size(m, n, k)
+    assert need > 0
+    for fmt, group, sdt in (("q8", 0, F32), ("q4g", 32, F32), ("q4g", 32, F16), ("q4g", 64, F32), ("q4g", 64, F16), ("q4g", 128, F32)):
+        t, gr = _make(nq, fmt, n, k, group, sdt, g)
+        for ydt in (F32, F16):
+            ws = torch.full((need,), 255, dtype=torch.uint8, device=dev)
+            y = torch.empty(m, n, dtype=ydt, device=dev)
+            _lib.check(_call(lib, x, t, y, ws, need, _lib.NQ_PATH_MFMA))
+            _check(y, x, _codes(t, gr), None, k)
+            assert bool((ws != 255).any()), (fmt, group, sdt, ydt)
+
+
 @gpu
 def test_less_workspace_splits_less(dev, nq):
     """The plain entries (no workspace) and a workspace below the preferred size give the
