@@ -29,7 +29,7 @@ nq_status wq_gemm(const XT* x, const uint8_t* w, const ST* sc, const float* b, Y
                   int64_t k, int64_t group, void* workspace, size_t workspace_bytes, hipStream_t s);
 size_t wq_workspace_bytes(int64_t m, int64_t n, int64_t k);
 bool wq_tile_route(bool q4, bool f32x, bool scale_f16, bool general, bool slices, int64_t m, int64_t n, int64_t k,
-                   int64_t group, bool ws);
+                   int64_t group, size_t ws_bytes);
 size_t wq_tile_ws_bytes(int64_t m, int64_t n, int64_t k);
 
 namespace {
@@ -2578,7 +2578,7 @@ nq_status linear_q8_impl(const void* x, nq_dtype x_dtype, const int8_t* q, const
     const TileCall tile{x_dtype == NQ_F32 ? TileX::F32 : TileX::F16, x, reinterpret_cast<const uint8_t*>(q), false, w_scale,
                         false, 0, nullptr, bias, y, y_dtype == NQ_F32 ? kTileF32 : kTileF16, m, n, k, !operands};
     if (path == NQ_PATH_AUTO && general && m <= 8 && tile_gemm_ok(false, m, n, k, 0)) return gemv_any(tile, s);
-    if (path == NQ_PATH_AUTO && wq_tile_route(false, x_dtype == NQ_F32, false, general, !operands, m, n, k, 0, ws != nullptr))
+    if (path == NQ_PATH_AUTO && wq_tile_route(false, x_dtype == NQ_F32, false, general, !operands, m, n, k, 0, ws ? ws_bytes : 0))
         return tile_gemm(tile, ws, ws_bytes, s);
     NQ_REQUIRE(!mfma || operands, NQ_BAD_ARG,
                "linear_q8: the MFMA path needs k %% 32 == 0 and 16-byte aligned x and q (m=%lld n=%lld k=%lld)",
@@ -2659,7 +2659,7 @@ nq_status linear_q4g_impl(const void* x, nq_dtype x_dtype, const uint8_t* q, con
                         bias, y, y_dtype == NQ_F32 ? kTileF32 : kTileF16, m, n, k, true};
     if (path == NQ_PATH_AUTO && general && m <= 8 && tile_gemm_ok(true, m, n, k, group)) return gemv_any(tile, s);
     if (path == NQ_PATH_AUTO && wq_tile_route(true, x_dtype == NQ_F32, scale_dtype == NQ_F16, general, !operands, m, n, k,
-                                              group, ws != nullptr))
+                                              group, ws ? ws_bytes : 0))
         return tile_gemm(tile, ws, ws_bytes, s);
     NQ_REQUIRE(!mfma || operands, NQ_BAD_ARG,
                "linear_q4g: the MFMA path needs k %% 32 == 0, group = 32 * 2^j and 16-byte aligned x and q "

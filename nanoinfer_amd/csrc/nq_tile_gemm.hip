@@ -792,8 +792,9 @@ size_t tile_gemm_ws_bytes(TileX xt, bool fine, int64_t m, int64_t n, int64_t k) 
 }
 
 bool tile_gemm_split_fits(TileX xt, bool fine, int64_t m, int64_t n, int64_t k, size_t ws_bytes) {
-    const int64_t have = static_cast<int64_t>(std::min<size_t>(ws_bytes, kTilePlanesMax));
-    return plan_tile(xt, fine, m, n, k, have).us <= 1.25 * plan_tile(xt, fine, m, n, k, kTilePlanesMax).us;
+    const TilePlan best = plan_tile(xt, fine, m, n, k, kTilePlanesMax);
+    if (best.splits < 2 || static_cast<size_t>(best.splits) * m * n * 4 <= ws_bytes) return true;
+    return plan_tile(xt, fine, m, n, k, static_cast<int64_t>(ws_bytes)).us <= (xt == TileX::F32 ? 1.15 : 1.05) * best.us;
 }
 
 nq_status tile_gemm(const TileCall& c, void* ws, size_t ws_bytes, hipStream_t s) {

@@ -29,7 +29,8 @@ bool tile_gemm_ok(bool q4, int64_t m, int64_t n, int64_t k, int64_t group);
 // Workspace its split-K planes take at this shape (0: no split); less or none is accepted
 // and splits less. fine: int4 codes, or TileCall::fine.
 size_t tile_gemm_ws_bytes(TileX xt, bool fine, int64_t m, int64_t n, int64_t k);
-// Whether the plan within ws_bytes comes within a quarter of the unlimited one.
+// Whether the plan within ws_bytes comes near the unlimited one: within 15% (F32) or 5%, as
+// past that the kernels with planes of their own are the faster ones on average.
 bool tile_gemm_split_fits(TileX xt, bool fine, int64_t m, int64_t n, int64_t k, size_t ws_bytes);
 nq_status tile_gemm(const TileCall& c, void* ws, size_t ws_bytes, hipStream_t s);
 

@@ -1165,9 +1165,11 @@ nq_status wq_gemm(const XT* x, const uint8_t* w, const ST* sc, const float* b, Y
 //   (1.6x); on it from m = 65 and k = 1024 up to 1.5 Mi outputs (1.2x), and on more where
 //   they would split K (m = 584, n = 8125, k = 5888 Q4G 162 -> 138); else the wide tiles win
 //   (m = 2048, n = 8960, k = 1536 Q8 56 against 96).
-// A call without a workspace keeps the other kernels where the tiles want to split K.
+// Where the tiles want to split K further than the workspace allows, the other kernels
+// keep the call, whose planes are in the required size (fp32 x, int8, with that: m = 24, n =
+// 512, k = 4096 7.5 against 11.5 on the tiles; m = 32, n = 256, k = 1536 7.6 against 11.2).
 bool wq_tile_route(bool q4, bool f32x, bool scale_f16, bool general, bool slices, int64_t m, int64_t n, int64_t k,
-                   int64_t group, bool ws) {
+                   int64_t group, size_t ws_bytes) {
     if (!tile_gemm_ok(q4, m, n, k, group)) return false;
     if (general) return m >= 9;
     const bool row = q4 && group >= k;
@@ -1187,10 +1189,10 @@ bool wq_tile_route(bool q4, bool f32x, bool scale_f16, bool general, bool slices
     } else {
         const bool sk64 = !q4 || group == 32;
         const bool few = m <= 128 && plan_wq_wide(m, n, sk64, false).tiles < 128;  // no wide tiles unsplit
-        const WqRoute r = plan_wq_route(m, n, k, !few, true, sk64, false, ws, q4);
+        const WqRoute r = plan_wq_route(m, n, k, !few, true, sk64, false, ws_bytes > 0, q4);
         take = !r.wide || (m >= 65 && (r.splits > 1 || m * n <= (int64_t(3) << 19)));
     }
-    return take && (ws || tile_gemm_split_fits(f32x ? TileX::F32 : TileX::F16, q4, m, n, k, 0));
+    return take && tile_gemm_split_fits(f32x ? TileX::F32 : TileX::F16, q4, m, n, k, ws_bytes);
 }
 
 // The split-K planes that the tile GEMM uses when the workspace holds them, for any

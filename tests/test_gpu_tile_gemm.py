@@ -263,6 +263,26 @@ def test_less_workspace_splits_less(dev, nq):
         assert float((y - full).norm() / full.norm()) < 1e-6
 
 
+@gpu
+@pytest.mark.parametrize("m,n,k", [(32, 128, 1024), (100, 128, 1536), (48, 128, 1024)])
+def test_required_workspace_keeps_the_kernel(dev, nq, m, n, k):
+    """With the required workspace only, of which the tile GEMM would need far more, fp32 rows
+    stay on the kernel whose planes that size holds (the explicit MFMA path, bit for bit)."""
+    from nanoinfer_amd import _lib
+    lib = _lib.load()
+    need, best = lib.nq_linear_wq_workspace_size(m, n, k), lib.nq_linear_wq_workspace_preferred(m, n, k)
+    assert 0 < need < best
+    ws = torch.empty(best, dtype=torch.uint8, device=dev)
+    x = torch.randn(m, k, device=dev)
+    for t, gr in (_make(nq, "q8", n, k, 0, F32, None), _make(nq, "q4g", n, k, 32, F32, None)):
+        y, ref = torch.empty(m, n, device=dev), torch.empty(m, n, device=dev)
+        _lib.check(_call(lib, x, t, ref, ws, need, _lib.NQ_PATH_MFMA))
+        _lib.check(_call(lib, x, t, y, ws, need, _lib.NQ_PATH_AUTO))
+        assert torch.equal(y, ref)
+        _lib.check(_call(lib, x, t, y, ws, best, _lib.NQ_PATH_AUTO))
+        _check(y, x, _codes(t, gr), None, k)
+
+
 def test_workspace_sizes_of_short_k():
     """Shapes below one 32-column chunk: no workspace is required (a division by the
     number of chunks once stood here)."""
