@@ -703,7 +703,7 @@ struct TilePlan {
     int cfg, splits;
     double us;  // modelled time
 };
-TilePlan plan_tile(TileX xt, bool fine, int64_t m, int64_t n, int64_t k, int64_t ws_bytes) {
+TilePlan model_plan(TileX xt, bool fine, int64_t m, int64_t n, int64_t k, int64_t ws_bytes) {
     const TileModel& mod = kTileModels[xt == TileX::I8 ? 4 : (xt == TileX::F16 ? 2 : 0) + (fine ? 1 : 0)];
     const int64_t sk = xt == TileX::F32 ? 32 : xt == TileX::F16 ? 64 : 128, slabs = (k + sk - 1) / sk;
     const double mn = static_cast<double>(m) * n;
@@ -724,6 +724,26 @@ TilePlan plan_tile(TileX xt, bool fine, int64_t m, int64_t n, int64_t k, int64_t
         }
     }
     return best;
+}
+
+// The plan of a shape, modelled once per thread while it stays among the last seen: a call
+// asks for up to six plans (each type's workspace, the route, the launch), 0.3 to 1 us each.
+TilePlan plan_tile(TileX xt, bool fine, int64_t m, int64_t n, int64_t k, int64_t ws_bytes) {
+    struct Seen {
+        int64_t m, n, k, ws;
+        int kind;
+        TilePlan plan;
+    };
+    constexpr unsigned kSeen = 64;
+    static thread_local Seen seen[kSeen];  // m = 0: empty
+    const int kind = static_cast<int>(xt) * 2 + (fine ? 1 : 0);
+    const uint64_t h = (static_cast<uint64_t>(m) * 0x9E3779B97F4A7C15u) ^ (static_cast<uint64_t>(n) * 0xC2B2AE3D27D4EB4Fu) ^
+                       (static_cast<uint64_t>(k) * 0x165667B19E3779F9u) ^ (static_cast<uint64_t>(ws_bytes) * 0xD6E8FEB86659FD93u) ^
+                       (static_cast<uint64_t>(kind) << 58);
+    Seen& e = seen[h >> 58];
+    if (e.m != m || e.n != n || e.k != k || e.ws != ws_bytes || e.kind != kind)
+        e = {m, n, k, ws_bytes, kind, model_plan(xt, fine, m, n, k, ws_bytes)};
+    return e.plan;
 }
 
 template <typename XT, WF F, int WM, int WN, int FM, int FN>
