@@ -832,7 +832,17 @@ nq_status run_gemm(const int8_t* xq, const float* as, const int8_t* wq, const fl
     const TileCall tile{TileX::I8, xq, reinterpret_cast<const uint8_t*>(wq), false, ws, false, 0, as, bias,
                         acc_out ? acc_out : y, acc_out ? kTileI32 : ydt == NQ_F32 ? kTileF32 : kTileF16, m, n, k, false};
     if (path == NQ_PATH_AUTO && m <= 8 && !mfma_ok(xq, wq, k) && tile_gemm_ok(false, m, n, k, 0)) return gemv_any(tile, s);
-    if (path == NQ_PATH_AUTO && w8a8_tile_route(mfma_ok(xq, wq, k), m, n, k)) return tile_gemm(tile, workspace, ws_bytes, s);
+    if (path == NQ_PATH_AUTO && w8a8_tile_route(mfma_ok(xq, wq, k), m, n, k)) {
+        // The shapes of the skinny kernel keep its conditions on the workspace; the others
+        // never had any, so a workspace that cannot hold planes is left alone.
+        const size_t need = mfma_ok(xq, wq, k) && skinny_ok(m, n, k) ? gemm_ws_bytes(m, n, k) : 0;
+        if (need) {
+            NQ_REQUIRE(workspace && ws_bytes >= need, NQ_BAD_ARG, "w8a8 gemm: workspace of %zu bytes required, %zu given",
+                       need, ws_bytes);
+            NQ_REQUIRE(aligned(workspace, 256), NQ_BAD_ALIGN, "w8a8 gemm: workspace must be 256-byte aligned");
+        }
+        return tile_gemm(tile, aligned(workspace, 256) ? workspace : nullptr, ws_bytes, s);
+    }
     if (p == NQ_PATH_MFMA && !mfma_ok(xq, wq, k)) p = NQ_PATH_GENERIC;
     // Weights past 2^31 bytes exceed the MFMA kernels' 32-bit buffer offsets;
     // the v_dot4 GEMV (64-bit addressing) takes them, in slices of 8 rows.

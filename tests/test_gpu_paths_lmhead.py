@@ -211,3 +211,34 @@ def test_nicpp_untied_without_lm_head_uses_embedding(tmp_path):
     assert mb.config.tie_word_embeddings == 0
     assert np.array_equal(ma.forward(PROMPT), mb.forward(PROMPT))
     assert ma.weight_bytes() == mb.weight_bytes()
+
+
+@pytest.mark.parametrize("m,n,k", [(130, 64, 8208), (200, 60, 16400), (200, 130, 4112), (200, 130, 1003), (40, 130, 4115)])
+def test_w8a8_codes_workspace(dev, nq, m, n, k):
+    """nq_gemm_w8a8 and nq_w8a8_acc_i32 past 128 rows off whole 64-column slabs: a short or
+    misaligned workspace is refused where one is required; where none is, one that cannot
+    hold planes is left alone."""
+    from nanoinfer_amd import _lib as L
+    lib = L.load()
+    g = torch.Generator(device=dev).manual_seed(k)
+    xq, wq = (torch.randint(-127, 128, (r, k), generator=g, device=dev, dtype=torch.int8) for r in (m, n))
+    a_s, w_s = torch.rand(m, generator=g, device=dev), torch.rand(n, generator=g, device=dev)
+    need, s = lib.nq_gemm_w8a8_workspace_size(m, n, k), torch.cuda.current_stream().cuda_stream
+    assert (need > 0) == (k >= 8192)
+    ws = torch.zeros((1 << 20) + max(need, lib.nq_gemm_w8a8_workspace_preferred(m, n, k)), dtype=torch.uint8, device=dev)
+    acc, y = torch.empty(m, n, dtype=torch.int32, device=dev), torch.empty(m, n, device=dev)
+
+    def both(off, nbytes):
+        p = ws.data_ptr() + off if nbytes else None
+        return (lib.nq_w8a8_acc_i32(xq.data_ptr(), wq.data_ptr(), acc.data_ptr(), m, n, k, p, nbytes, 0, s),
+                lib.nq_gemm_w8a8(xq.data_ptr(), a_s.data_ptr(), wq.data_ptr(), w_s.data_ptr(), None, y.data_ptr(), 0, m, n, k, p,
+                                 nbytes, 0, s))
+
+    bad_arg, bad_align = 4, 2
+    ref = xq.double() @ wq.double().t().contiguous()
+    for off, nbytes, refused in ((0, 0, bad_arg), (0, need - 1, bad_arg), (64, need + 256, bad_align), (0, need, 0)) if need else (
+            (0, 0, 0), (1, 1 << 20, 0), (64, 1 << 20, 0), (0, 1 << 20, 0)):
+        assert both(off, nbytes) == (refused, refused), (off, nbytes)
+        if not refused:
+            assert torch.equal(acc.double(), ref)
+            assert float((y.double() - ref * a_s.double()[:, None] * w_s.double()).abs().max()) <= 2.0 ** -22 * float(ref.abs().max())
