@@ -74,7 +74,7 @@ PyObject* call(Py_ssize_t n, F f) {
     try {
         const int device = c10::hip::current_device();
         r = f(device, c10::hip::getCurrentHIPStream(static_cast<c10::DeviceIndex>(device)).stream());
-    } catch (const std::exception&) {
+    } catch (...) {
         r = nullptr;
     }
     if (PyErr_Occurred()) PyErr_Clear();
@@ -82,14 +82,16 @@ PyObject* call(Py_ssize_t n, F f) {
     Py_RETURN_NONE;
 }
 
-// The library call without the interpreter lock, as ctypes makes it.
+// The library call without the interpreter lock, as ctypes makes it. What f throws (a
+// tensor that gives no data pointer) finds the lock held again.
+struct Unlocked {
+    PyThreadState* const state = PyEval_SaveThread();
+    ~Unlocked() { PyEval_RestoreThread(state); }
+};
 template <typename F>
 bool launch(F f) {
-    nq_status st;
-    Py_BEGIN_ALLOW_THREADS;
-    st = f();
-    Py_END_ALLOW_THREADS;
-    return st == NQ_OK;
+    const Unlocked unlocked;
+    return f() == NQ_OK;
 }
 
 PyObject* wrap(at::Tensor t) { return THPVariable_Wrap(std::move(t)); }

@@ -62,6 +62,46 @@ def test_same_as_python_path(dev, nq, declined, dt, m, n, k):
         _same(y, ref)
 
 
+def test_on_the_current_stream(dev, nq):
+    """The launches queue on the current stream: behind a delay there, a copy into the input
+    comes first. (Launched on any other stream they would read the old input.)"""
+    from nanoinfer_amd import model
+    m, k = 24, 512
+    g = torch.Generator(device=dev).manual_seed(1)
+    new = lambda *s: torch.randn(*s, generator=g, device=dev)
+    t8, t4, h = nq.quantize_q8(new(300, k)), nq.quantize_q4g(new(300, k), 32), new(k)
+    cos, sin = new(64, 64), new(64, 64)
+    heads = lambda x: x.view(4, m, k // 4)
+    calls = [lambda x: nq.linear_q8(x, t8), lambda x: nq.linear_q4g(x, t4), lambda x: nq.linear_w8a8(x, t8),
+             lambda x: nq.gemm_w8a8(*nq.act_quant(x), t8), nq.act_quant, lambda x: nq.act_quant_heads(heads(x)),
+             lambda x: nq.rmsnorm_quant(x, h, 1e-6), lambda x: nq.add_rmsnorm_quant(x, x, h, 1e-6),
+             lambda x: nq.silu_mul_quant(x[:, :k // 2], x[:, k // 2:]), lambda x: nq._calls.silu_mul_quant(x, None),
+             lambda x: model.rope_qkv(x, 4, 2, 64, cos, sin), lambda x: model.attention(*[x.view(8, m, 64)] * 3, 1),
+             lambda x: (lambda t: (t.q, t.scale))(nq.quantize_q8(x)), lambda x: (lambda t: (t.q, t.scale))(nq.quantize_q4g(x, 32))]
+    side = torch.cuda.Stream()
+    for i, f in enumerate(calls):
+        dt = torch.float16 if i in (2, 11) else torch.float32
+        old, other = new(m, k).to(dt), new(m, k).to(dt)
+        ref = f(other)
+        x = old.clone()
+        torch.cuda.synchronize()
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(10_000_000)
+            x.copy_(other)
+            y = f(x)
+        side.synchronize()
+        _same(y, ref)
+
+
+def test_data_pointer_that_throws(dev, nq):
+    """A tensor without a data pointer: an error, from every call that asks for one."""
+    x, t = torch.randn(4, 64, device=dev), nq.quantize_q8(torch.randn(16, 64, device=dev))
+    torch._C._set_throw_on_mutable_data_ptr(x)
+    for f in (lambda: nq.linear_q8(x, t), lambda: nq.linear_w8a8(x, t), lambda: nq.act_quant(x), lambda: nq.quantize_q8(x)):
+        with pytest.raises(RuntimeError):
+            f()
+
+
 class Sub(torch.Tensor):
     pass
 
