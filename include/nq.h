@@ -42,8 +42,8 @@ typedef enum nq_status {
 typedef enum nq_dtype { NQ_F32 = 0, NQ_F16 = 1 } nq_dtype;
 
 /* Kernel selection for the W8A8 linears. AUTO: operands that fit neither the GEMVs nor the
- * MFMA kernels (k % 16, alignment), from m = 9, and k % 64 past m = 128 -> the tile GEMM over
- * any k; else m <= 4 (m <= 8 when k >= 4096 or n >= 8192)
+ * MFMA kernels (k % 16, alignment), from m = 9, and k % 64 past m = 128 on long K or from
+ * 0.7 G products -> the tile GEMM over any k; else m <= 4 (m <= 8 when k >= 4096 or n >= 8192)
  * -> workgroup-per-rows GEMV (v_dot4_i32_i8), larger m -> int8 MFMA GEMM; nq_linear_w8a8 runs
  * m = 1 as one GEMV launch with the act quant fused in, and with AUTO tries the one-launch
  * decode kernel (m * k <= 4096, or m <= 4 and m * k <= 8192) and the decode kernel over the act quant's codes

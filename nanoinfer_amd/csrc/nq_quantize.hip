@@ -18,7 +18,7 @@ constexpr int kRowThreads = 256;
 
 // One workgroup per row: absmax over the row (block reduction through LDS),
 // scale = absmax / 127, then each thread quantizes its strided elements.
-// Rows that the vector kernel below does not take (fewer than 8 elements, or over 65536).
+// Rows that the vector kernel below does not take (short ones off 8 elements, or over 65536).
 template <typename XT>
 __global__ __launch_bounds__(kRowThreads) void quantize_rows_i8_kernel(
     const XT* __restrict__ x, int8_t* __restrict__ q, float* __restrict__ scale, int k) {
@@ -164,7 +164,7 @@ __global__ void quantize_q4g_odd_kernel(const float* __restrict__ w, uint8_t* __
 // ---- activation quant (vectorized) ------------------------------
 // One workgroup per row, 8 elements per 16-byte step (fp16) held in registers between
 // the absmax pass and the quantize pass (x is read once), at whatever address the row
-// starts; the last k % 8 elements go one to a thread. Rows off 8 elements took two
+// starts; the last k % 8 elements go one to a thread. Long rows off 8 elements took two
 // passes of single elements (us: m = 2048, k = 1003 fp16 8.3 -> 7.3; m = 512, k = 8955
 // 16.5 -> 8.7; weights of 9000 x 9001 181 -> 75).
 // HEADS: x is head-major [k / hd, m, hd] (an attention output) and row `row`
@@ -242,7 +242,10 @@ nq_status act_quant(const void* x, nq_dtype xdt, int64_t m, int64_t k, int8_t* x
     // One workgroup per row: for m >= 256, 256 threads with up to 8 vectors of
     // 8 elements each (k <= 16384; several vectors per thread keep more loads
     // in flight and let several rows share a CU), else 1024 threads with up to 8.
-    const bool vec = k >= 8 && k <= 8 * 1024 * 8;
+    // Short rows off 8 elements stay on single elements, whose two passes over at most three
+    // elements a thread are shorter (us, elements / vectors: m = 1892, k = 114 fp16 3.7 / 4.7; m =
+    // 1301, k = 364 1.09 times; from k = 640 the vectors win, k = 1028 0.90, k = 1773 0.77).
+    const bool vec = k <= 8 * 1024 * 8 && (k % 8 == 0 && aligned(x, 16) && aligned(xq, 8) ? k > 0 : k >= 640);
     if (vec) {
         const unsigned grid = static_cast<unsigned>(m);
         const int64_t steps = k / 8;
@@ -364,7 +367,8 @@ extern "C" nq_status nq_quantize_q4g(const float* w, int64_t out, int64_t in, in
     const int threads = 256;
     hipStream_t s = as_stream(stream);
     const int gl = g / 8;  // lanes per block on the vector path
-    if (g % 8 == 0 && gl <= 64 && (gl & (gl - 1)) == 0) {
+    // Under 8 columns the element kernels win (n = 1985, k = 3, groups of 128 3.3 / 4.2 us).
+    if (g % 8 == 0 && gl <= 64 && (gl & (gl - 1)) == 0 && k >= 8) {
         const int cpr = (((k + 7) / 8 + gl - 1) / gl) * gl;
         const unsigned grid = static_cast<unsigned>((out * cpr + 255) / 256);
         auto go = [&](auto gtag, auto* sp) {

@@ -812,12 +812,15 @@ int resolve_path(int path, int64_t m, int64_t n, int64_t k) {
 // Whether AUTO runs the tile GEMM (nq_tile_gemm.hip): from m = 9 where the operands fit
 // neither the MFMA kernels nor the GEMVs (k % 16, alignment; us, wave per row -> this:
 // m = 40, n = 1001, k = 1003 68 -> 8.2; m = 128, n = 4864, k = 900 264 -> 9.2), and past
-// 128 rows where k % 64 keeps the wide tiles away (the skinny kernel over 64-row
-// blocks: m = 1122, n = 1336, k = 5488 69 -> 32; 1.1x at m <= 512, 2.1x above). Its
-// int32 sums are exact, so the results are the other paths' bit for bit.
+// 128 rows where k % 64 keeps the wide tiles away, from k = 800 and 0.7 G products or k =
+// 4000 (the skinny kernel over 64-row blocks -> this: m = 1122, n = 1336, k = 5488 69 ->
+// 32; m = 212, n = 2217, k = 1648 13.6 -> 9.7; short of that the skinny kernel wins, m = 500, n
+// = 1057, k = 352 5.9 against 9.3, m = 1867, n = 5435, k = 272 31 against 42). Its int32
+// sums are exact, so the results are the other paths' bit for bit.
 bool w8a8_tile_route(bool operands_ok, int64_t m, int64_t n, int64_t k) {
     if (!tile_gemm_ok(false, m, n, k, 0)) return false;
-    return operands_ok ? m > 128 && k % kBK != 0 : m >= 9;
+    if (!operands_ok) return m >= 9;
+    return m > 128 && k % kBK != 0 && (k >= 4000 || (k >= 800 && m * n * k >= 700000000));
 }
 size_t w8a8_tile_ws_bytes(int64_t m, int64_t n, int64_t k) {
     if (!w8a8_tile_route(k > 0 && k % 16 == 0, m, n, k)) return 0;

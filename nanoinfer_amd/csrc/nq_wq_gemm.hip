@@ -1157,14 +1157,22 @@ nq_status wq_gemm(const XT* x, const uint8_t* w, const ST* sc, const float* b, Y
 //   10^4 times; m = 40, n = 1001, k = 1003: Q8 82 -> 8.8, Q4G 138 -> 8.9; m = 1500, n =
 //   6768, k = 2160: Q8 2146 -> 90, one int4 group per row 6 * 10^5 -> 88, a lane per group);
 //   from m = 16 where only the GEMVs do, in slices of 8 rows (`slices`; one int4 group per
-//   row, seldom a power of two of chunks, 10x), and for one group per row throughout,
-//   except fp16 x past m = 512 on the wide tiles' contract;
+//   row, seldom a power of two of chunks, 10x; up to 31 rows if the K split fits the
+//   workspace: m = 17, n = 1344, k = 1536, fp32, one group 13.4 against 23.4 without);
 //   fp32 x from m = 32 and k = 512 (2.8x; m = 333, n = 1536, k = 8960 Q8 85 -> 45), and from
-//   m = 16 on k >= 1024 and 512 weight rows (1.5x); shorter K loses up to 1.3x;
+//   m = 16 on 512 weight rows and k = 1024, or 2048 rows and k = 2048 (m = 20, n = 7424, k =
+//   1664 Q4G 13.4 against 16.3). Up to 63 rows not on k < 1024 with 1024 to 4095 weight rows
+//   (m = 39, n = 3648, k = 512 Q8 6.8 against 9.5), nor on long K with few weight rows,
+//   where the old kernels split K further: under 1024, k >= 3584 (m = 24, n = 512, k = 4096 Q8
+//   7.5 against 8.8), but under 400 on the wide tiles' contract, and 400 or more off it from
+//   m = 32, the tiles win (0.83 and 0.81 of the time);
 //   fp16 x off the wide tiles' contract, or too few of them, from m = 33 and k = 1024
-//   (1.6x); on it from m = 65 and k = 1024 up to 1.5 Mi outputs (1.2x), and on more where
-//   they would split K (m = 584, n = 8125, k = 5888 Q4G 162 -> 138); else the wide tiles win
-//   (m = 2048, n = 8960, k = 1536 Q8 56 against 96).
+//   (1.6x; short of m = 48 and k = 1536 not on 2048 to 4095 weight rows: m = 43, n = 3392, k =
+//   1024 Q4G 7.8 against 9.7); on it from m = 65 and k = 1024 up to 1.5 Mi outputs (1.2x), and
+//   on more where they would split K (m = 584, n = 8125, k = 5888 Q8 162 -> 138), but int4 in
+//   groups past 128 rows only up to 1023 weight rows, and past 255 up to 511 (m = 333, n =
+//   1536, k = 8960 groups of 64 32.9 against 39.1); else the wide tiles win (m = 2048, n =
+//   8960, k = 1536 Q8 56 against 96).
 // Where the tiles want to split K further than the workspace allows, the other kernels
 // keep the call, whose planes are in the required size (fp32 x, int8, with that: m = 24, n =
 // 512, k = 4096 7.5 against 11.5 on the tiles; m = 32, n = 256, k = 1536 7.6 against 11.2).
@@ -1172,16 +1180,16 @@ bool wq_tile_route(bool q4, bool f32x, bool scale_f16, bool general, bool slices
                    int64_t group, size_t ws_bytes) {
     if (!tile_gemm_ok(q4, m, n, k, group)) return false;
     if (general) return m >= 9;
-    const bool row = q4 && group >= k;
+    if (slices) return m >= 32 || (m >= 16 && tile_gemm_split_fits(f32x ? TileX::F32 : TileX::F16, true, m, n, k, ws_bytes));
     bool wide;
     if (!q4) wide = f32x ? wq_wide_contract<false, float, float>(m, n, k, 32) : wq_wide_contract<false, _Float16, float>(m, n, k, 32);
     else if (f32x) wide = wq_wide_contract<true, float, float>(m, n, k, group);
     else wide = scale_f16 ? wq_wide_contract<true, _Float16, _Float16>(m, n, k, group) : wq_wide_contract<true, _Float16, float>(m, n, k, group);
-    wide = wide && !slices;
-    if (m >= 16 && (slices || (row && (f32x || m <= 512 || !wide)))) return true;
     bool take;
     if (f32x) {
-        take = (m >= 32 && k >= 512) || (m >= 16 && k >= 1024 && n >= 512);
+        if (m < 32) take = m >= 16 && n >= 512 && k >= (n < 2048 ? 1024 : 2048);
+        else take = k >= 1024 || (k >= 512 && (m >= 64 || n < 1024 || n >= 4096));
+        if (m < 64 && n < 1024 && k >= 3584 && (wide ? n >= 400 : m < 32 || n < 400)) take = false;
     } else if (m < 33 || k < 1024) {
         take = false;
     } else if (!wide) {
@@ -1190,7 +1198,8 @@ bool wq_tile_route(bool q4, bool f32x, bool scale_f16, bool general, bool slices
         const bool sk64 = !q4 || group == 32;
         const bool few = m <= 128 && plan_wq_wide(m, n, sk64, false).tiles < 128;  // no wide tiles unsplit
         const WqRoute r = plan_wq_route(m, n, k, !few, true, sk64, false, ws_bytes > 0, q4);
-        take = !r.wide || (m >= 65 && (r.splits > 1 || m * n <= (int64_t(3) << 19)));
+        if (!r.wide) take = m >= 48 || k >= 1536 || n < 2048 || n >= 4096;
+        else take = m >= 65 && (r.splits > 1 || m * n <= (int64_t(3) << 19)) && (!q4 || m <= 128 || n < (m < 256 ? 1024 : 512));
     }
     return take && tile_gemm_split_fits(f32x ? TileX::F32 : TileX::F16, q4, m, n, k, ws_bytes);
 }

@@ -120,7 +120,7 @@ def test_q8_of_whole_chunks(dev, nq, xdt, m, n, k):
 def test_errors_on_long_k(dev, nq, xdt, fmt, group):
     g = torch.Generator(device=dev).manual_seed(group)
     lim = 2.0 ** -24 * ((9.5 if xdt == F32 else 6.5) / 3) ** 0.5
-    for m, n, k in ((4, 200, 8955), (8, 2100, 1003), (12, 256, 1003), (130, 515, 8955),
+    for m, n, k in ((2, 8194, 301), (3, 8195, 149), (4, 200, 8955), (8, 2100, 1003), (12, 256, 1003), (130, 515, 8955),
                     (333, 4500, 8960 if fmt == "q4" else 9001), (600, 4001, 1003)):
         t, gr = _make(nq, fmt, n, k, group, F32, g)
         x = torch.randn(m, k, generator=g, device=dev).to(xdt)
@@ -281,6 +281,30 @@ def test_required_workspace_keeps_the_kernel(dev, nq, m, n, k):
         assert torch.equal(y, ref)
         _lib.check(_call(lib, x, t, y, ws, best, _lib.NQ_PATH_AUTO))
         _check(y, x, _codes(t, gr), None, k)
+
+
+# Calls that the tile GEMM or the GEMVs of any k are slower for: bit for bit the kernels of
+# the explicit paths.
+@gpu
+@pytest.mark.parametrize("xdt,m,n,k,fmt,group", [
+    (F32, 39, 3648, 512, "q8", 0), (F32, 20, 7424, 1664, "q4g", 32), (F32, 24, 512, 4096, "q8", 0), (F32, 46, 256, 7168, "q4g", 64),
+    (F32, 20, 512, 256, "q4", 0), (F16, 19, 320, 512, "q4", 0), (F16, 43, 3392, 1024, "q4g", 32), (F16, 333, 1536, 8960, "q4g", 64)])
+def test_kept_on_mfma(dev, nq, xdt, m, n, k, fmt, group):
+    from nanoinfer_amd import _lib
+    t, gr = _make(nq, fmt, n, k, group, F32, None)
+    x = torch.randn(m, k, device=dev).to(xdt)
+    f = nq.linear_q8 if fmt == "q8" else nq.linear_q4g
+    assert torch.equal(f(x, t), f(x, t, path=_lib.NQ_PATH_MFMA))
+
+
+@gpu
+@pytest.mark.parametrize("xdt", [F32, F16])
+@pytest.mark.parametrize("m,n,k", [(1, 2358, 65), (2, 6462, 87), (2, 60, 255), (5, 426, 51), (8, 90, 111)])
+def test_kept_on_elements(dev, nq, xdt, m, n, k):
+    from nanoinfer_amd import _lib
+    t, _ = _make(nq, "q8", n, k, 0, F32, None)
+    x = torch.randn(m, k, device=dev).to(xdt)
+    assert torch.equal(nq.linear_q8(x, t), nq.linear_q8(x, t, path=_lib.NQ_PATH_GENERIC))
 
 
 def test_workspace_sizes_of_short_k():
