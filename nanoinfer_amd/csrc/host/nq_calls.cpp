@@ -300,9 +300,13 @@ PyObject* attention(PyObject*, PyObject* const* a, Py_ssize_t n) {
             if (t->t->dim() != 3 || t->t->scalar_type() != at::kHalf || t->t->unsafeGetTensorImpl()->autograd_meta() != nullptr)
                 return nullptr;
         const int64_t h = q.size(0), rows = q.size(1), d = q.size(2), kv = k.size(0);
-        if ((d != 64 && d != 128) || k.t->sizes() != v.t->sizes() || k.size(1) != rows || k.size(2) != d || kv < 1 || h < 1 || h % kv ||
-            rows > (d == 64 ? 1024 : 2048))  // measured up to here: longer rows are torch's
+        if ((d != 64 && d != 128) || k.t->sizes() != v.t->sizes() || k.size(1) != rows || k.size(2) != d || kv < 1 || h < 1 || h % kv)
             return nullptr;
+        // Longer rows are torch's, unmeasured, and so are many heads of long ones: 16 queries to each
+        // read of K and V bound this kernel once its workgroups fill the GPU (us, this / torch: 28 heads
+        // of 128, 768 tokens 40 / 44, 1024 64 / 55; 16 heads, 1536 73 / 84, 2048 112 / 104; 64 heads, 512
+        // 46 / 40; heads of 64: 32, 768 tokens 30 / 31, 1024 45 / 38).
+        if (rows > (d == 64 ? 1024 : 2048) || h * rows > 24576) return nullptr;
         const at::Tensor out = empty({h, rows, d}, at::kHalf, dev);
         const bool ok = launch([&] { return nq_attention_causal_f16(q.p(), k.p(), v.p(), h, kv, rows, d, out.data_ptr(), s); });
         return ok ? wrap(out) : nullptr;

@@ -64,6 +64,11 @@ def test_calls_that_stay_with_torch(dev):
     assert c(q[:3].contiguous(), k, v) is None and c(q[..., :32].contiguous(), k[..., :32].contiguous(), v[..., :32].contiguous()) is None
     long = torch.zeros(2, 1025, 64, device=dev).half()
     assert c(long, long, long) is None and c(long[:, :1024].contiguous(), *[long[:, :1024].contiguous()] * 2) is not None
+    for d, h, s, ours in ((128, 32, 768, True), (128, 32, 769, False), (128, 12, 2048, True), (128, 13, 2048, False),
+                          (64, 24, 1024, True), (64, 25, 1024, False)):
+        t = torch.zeros(h, s, d, device=dev).half()
+        assert (c(t, t, t) is not None) == ours
+        assert model.attention(t, t, t, 1).shape == t.shape
     qg = q.clone().requires_grad_()
     y = model.attention(qg, k, v, 2)
     y.float().sum().backward()
