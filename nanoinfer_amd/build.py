@@ -75,9 +75,22 @@ def _host_artifacts():
           "-I", sysconfig.get_paths()["include"], "-o", mod + ".tmp", os.path.join(host_src, "nicpp.cpp"),
           "-L", PKG, "-lnq_host", "-lnq_hip", rpath], "nicpp module")
     os.replace(mod + ".tmp", mod)
-    # _calls: the native call path of quant.py, on torch's own tensors and allocator.
-    import torch
+    _run([*cxx, "-o", HOST_TEST + ".tmp", os.path.join(ROOT, "tests", "cpp", "test_host.cpp"),
+          "-L", PKG, "-lnq_host", "-lnq_hip", "-Wl,-rpath," + PKG, "-Wl,-rpath,$ORIGIN/../../nanoinfer_amd"],
+         "C++ host test")
+    os.replace(HOST_TEST + ".tmp", HOST_TEST)
+    return [HOST_LIB, mod, HOST_TEST, *_torch_calls(cxx, host_src, rpath, ext)]
 
+
+def _torch_calls(cxx, host_src, rpath, ext):
+    """_calls: the native call path of quant.py, on torch's own tensors and allocator. Nothing
+    above it needs torch, so where torch is missing only quant.py's layer is."""
+    import sysconfig
+
+    try:
+        import torch
+    except ImportError:
+        return []
     troot = os.path.dirname(torch.__file__)
     calls = os.path.join(PKG, "_calls" + ext)
     _run([*cxx, "-shared", "-fvisibility=hidden", "-DUSE_ROCM", "-D__HIP_PLATFORM_AMD__",
@@ -87,11 +100,7 @@ def _host_artifacts():
           "-L", PKG, "-lnq_hip", "-L", os.path.join(troot, "lib"), "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip", rpath],
          "_calls module")
     os.replace(calls + ".tmp", calls)
-    _run([*cxx, "-o", HOST_TEST + ".tmp", os.path.join(ROOT, "tests", "cpp", "test_host.cpp"),
-          "-L", PKG, "-lnq_host", "-lnq_hip", "-Wl,-rpath," + PKG, "-Wl,-rpath,$ORIGIN/../../nanoinfer_amd"],
-         "C++ host test")
-    os.replace(HOST_TEST + ".tmp", HOST_TEST)
-    return [HOST_LIB, mod, calls, HOST_TEST]
+    return [calls]
 
 
 def build(verbose: bool = False) -> str:
