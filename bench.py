@@ -173,7 +173,7 @@ def main():
         qs = [t.q] + [t.q.clone() for _ in range(copies_for(wbytes) - 1)]
         ss = [t.scale] + [t.scale.clone() for _ in range(len(qs) - 1)]
         y = torch.empty((m, n), dtype=torch.float16, device=dev)
-        wsb = lib.nq_linear_wq_workspace_size(m, n, k)  # split-K planes (0: none)
+        wsb = lib.nq_linear_wq_workspace_preferred(m, n, k)  # split-K planes (0: none)
         work = torch.empty(max(wsb, 256), dtype=torch.uint8, device=dev) if wsb else None
 
         def mk(i):
@@ -193,7 +193,7 @@ def main():
         ss = [t.scale] + [t.scale.clone() for _ in range(len(qs) - 1)]
         y = torch.empty((m, n), dtype=xdt, device=dev)
         dt = 1 if xdt == torch.float16 else 0
-        wsb = lib.nq_linear_wq_workspace_size(m, n, k)
+        wsb = lib.nq_linear_wq_workspace_preferred(m, n, k)
         work = torch.empty(max(wsb, 256), dtype=torch.uint8, device=dev) if wsb else None
 
         def mk(i):
@@ -255,14 +255,14 @@ def main():
         y = torch.empty((m, n), dtype=torch.float16, device=dev)
         if gemm_only:
             xq, a_s = nq.act_quant(x)
-            wsb = lib.nq_gemm_w8a8_workspace_size(m, n, k)
+            wsb = lib.nq_gemm_w8a8_workspace_preferred(m, n, k)
             ws = torch.empty(max(wsb, 256), dtype=torch.uint8, device=dev)
 
             def mk(i):
                 return lambda: lib.nq_gemm_w8a8(P(xq), P(a_s), P(qs[i]), P(ss[i]), None, P(y), 1, m, n, k,
                                                 P(ws), ws.numel(), 0, stream_ptr())
         else:
-            wsb = lib.nq_linear_w8a8_workspace_size(m, n, k)
+            wsb = lib.nq_linear_w8a8_workspace_preferred(m, n, k)
             ws = torch.empty(max(wsb, 256), dtype=torch.uint8, device=dev)
 
             def mk(i):
@@ -557,9 +557,8 @@ def decoder_layer_cfg4(rnd, time_graph, args, w8a8_linear, entry):
     proj_ops = sum(2 * m * o * i for o, i in shapes.values())
     del mdl
     torch.cuda.empty_cache()
-    # The layer's causal GQA attention is torch's scaled_dot_product_attention
-    # (AOTriton on ROCm), outside this path: timed alone at the layer's shape and
-    # reported as non-product time.
+    # The layer's causal GQA attention, no part of the quantized path: timed alone at the
+    # layer's shape.
     hq = torch.randn((cfg.heads, m, cfg.head_dim), device="cuda").half()
     hk = torch.randn((cfg.kv_heads, m, cfg.head_dim), device="cuda").half()
     hv = torch.randn((cfg.kv_heads, m, cfg.head_dim), device="cuda").half()
@@ -568,11 +567,10 @@ def decoder_layer_cfg4(rnd, time_graph, args, w8a8_linear, entry):
     del hq, hk, hv
     e = {"name": f"decoder_layer_cfg4 M={m} Qwen2.5-1.5B: the 7 W8A8 projections (4 fused GEMMs on this path)",
          "layer_us": round(ms * 1e3, 3), "layers_chained": L,
-         "layer_note": "whole layer: projections + fused act quants + RoPE (this path) + torch SDPA attention "
-                       "(non-product)",
+         "layer_note": "whole layer: projections + fused act quants + RoPE + attention",
          "attention_us_nonproduct": round(attn_ms * 1e3, 3),
-         "attention_note": "torch.nn.functional.scaled_dot_product_attention (AOTriton attn_fwd on ROCm), "
-                           "timed alone at the layer's shape; not part of the quantized path"}
+         "attention_note": "model.attention (attention_causal_f16_kernel), timed alone at the layer's shape; not "
+                           "part of the quantized path"}
     torch.cuda.empty_cache()
     # The layer runs q|k|v and gate|up as fused GEMMs on pre-quantized input
     # (activation quant fused into rmsnorm / silu*up); these are timed as GEMMs.

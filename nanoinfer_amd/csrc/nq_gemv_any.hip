@@ -13,9 +13,9 @@
 //
 // Bound by latency on small weights and by the activation re-reads (one per R weight
 // rows) at 8 rows. us, element kernel -> this: Q8 fp32 x, n = 1001, k = 1003 m = 7 15.4 ->
-// 5.1; n = 1536, k = 8955 m = 1 37 -> 7.9, m = 8 272 -> 17; n = k = 9001 m = 2 146 -> 26
-// (3.1 TB/s); Q4G m = 1, n = 17920, k = 1531 83 -> 13; one int4 group per row, m = 8, n =
-// 1536, k = 8955 7029 -> 13; W8A8 m = 2, n = k = 9001 135 -> 19 (4.2 TB/s).
+// 6.1; n = 1536, k = 8955 m = 1 37 -> 6.7, m = 8 272 -> 14; n = k = 9001 m = 2 146 -> 26
+// (3.1 TB/s); Q4G m = 1, n = 17920, k = 1531 83 -> 9.2; one int4 group per row, m = 8, n =
+// 1536, k = 8955 7029 -> 13; W8A8 m = 2, n = k = 9001 135 -> 17 (4.7 TB/s).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -173,7 +173,8 @@ void launch_any(AnyArgs a, hipStream_t s) {
     // Two weight rows per wave; four from 8192 rows, which leave waves enough for half the
     // activation re-reads.
     const int R = a.n >= 8192 ? 4 : 2;
-    // K over 2 or 4 waves while rows alone leave under 4096 waves, with 64 pieces of 16 each.
+    // K over 2 or 4 waves while rows alone leave under 4096 waves, with at least 1024 columns
+    // each: 64 pieces of 16, or 128 of 8.
     const int waves = (a.n + R - 1) / R;
     a.kw = a.k >= 4096 && waves < 2048 ? 4 : a.k >= 2048 && waves < 4096 ? 2 : 1;
     const int rows = R * 4 / a.kw;

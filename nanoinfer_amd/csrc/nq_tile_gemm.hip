@@ -676,7 +676,8 @@ __global__ __launch_bounds__(256) void tile_reduce_kernel(TileArgs a, int splits
 // than it has (first loads, stores); a split adds a launch and the planes' traffic.
 // Least-squares fit to the measured (shape, tile, split) points of 5400 shapes (m
 // 5..2048, n 128..18432, k 1..9216): the pick is 1.5% slower than the measured best on
-// average, 5% at the 90th percentile.
+// average, 5% at the 90th percentile. The points of the fine sums' rows are int4 groups with
+// fp32 sums of the parts; with fp64 ones the larger tiles take up to a fifth longer.
 struct TileCost {
     float extra, alone, shared;
 };

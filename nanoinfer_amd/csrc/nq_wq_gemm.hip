@@ -1154,8 +1154,8 @@ nq_status wq_gemm(const XT* x, const uint8_t* w, const ST* sc, const float* b, Y
 // old -> new, measured over 1780 shapes):
 //   from m = 9 where no kernel here nor any GEMV takes the operands (`general`: k %
 //   16 or 32, alignment, groups), which fell to a wave per row (all of 250 shapes, 1.1 to
-//   10^4 times; m = 40, n = 1001, k = 1003: Q8 82 -> 8.8, Q4G 138 -> 8.9; m = 1500, n =
-//   6768, k = 2160: Q8 2146 -> 90, one int4 group per row 6 * 10^5 -> 88, a lane per group);
+//   10^4 times; m = 40, n = 1001, k = 1003: Q8 82 -> 9.7, Q4G 138 -> 10; m = 1500, n =
+//   6768, k = 2160: Q8 2146 -> 105, one int4 group per row 6 * 10^5 -> 94, a lane per group);
 //   from m = 16 where only the GEMVs do, in slices of 8 rows (`slices`; one int4 group per
 //   row, seldom a power of two of chunks, 10x; up to 31 rows if the K split fits the
 //   workspace: m = 17, n = 1344, k = 1536, fp32, one group 13.4 against 23.4 without);
@@ -1169,10 +1169,9 @@ nq_status wq_gemm(const XT* x, const uint8_t* w, const ST* sc, const float* b, Y
 //   fp16 x off the wide tiles' contract, or too few of them, from m = 33 and k = 1024
 //   (1.6x; short of m = 48 and k = 1536 not on 2048 to 4095 weight rows: m = 43, n = 3392, k =
 //   1024 Q4G 7.8 against 9.7); on it from m = 65 and k = 1024 up to 1.5 Mi outputs (1.2x), and
-//   on more where they would split K (m = 584, n = 8125, k = 5888 Q8 162 -> 138), but int4 in
-//   groups past 128 rows only up to 1023 weight rows, and past 255 up to 511 (m = 333, n =
-//   1536, k = 8960 groups of 64 32.9 against 39.1); else the wide tiles win (m = 2048, n =
-//   8960, k = 1536 Q8 56 against 96).
+//   on more where they would split K, but int4 past 128 rows only up to 1023 weight rows, and
+//   past 255 up to 511 (m = 333, n = 1536, k = 8960 groups of 64 32.9 against 39.1); else the
+//   wide tiles win (m = 2048, n = 8960, k = 1536 Q8 56 against 96).
 // Where the tiles want to split K further than the workspace allows, the other kernels
 // keep the call, whose planes are in the required size (fp32 x, int8, with that: m = 24, n =
 // 512, k = 4096 7.5 against 11.5 on the tiles; m = 32, n = 256, k = 1536 7.6 against 11.2).
