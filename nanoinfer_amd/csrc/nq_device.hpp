@@ -167,6 +167,15 @@ __device__ __forceinline__ T swap_sum(T a, T b) {
     const SwapPair r = row_swap<O>(__builtin_bit_cast(unsigned, a), __builtin_bit_cast(unsigned, b));
     return __builtin_bit_cast(T, r.first) + __builtin_bit_cast(T, r.second);
 }
+// Doubles move as their two dwords.
+template <int O>
+__device__ __forceinline__ double swap_sum(double a, double b) {
+    const uint64_t x = __builtin_bit_cast(uint64_t, a), y = __builtin_bit_cast(uint64_t, b);
+    const SwapPair l = row_swap<O>(static_cast<unsigned>(x), static_cast<unsigned>(y));
+    const SwapPair h = row_swap<O>(static_cast<unsigned>(x >> 32), static_cast<unsigned>(y >> 32));
+    return __builtin_bit_cast(double, static_cast<uint64_t>(h.first) << 32 | l.first) +
+           __builtin_bit_cast(double, static_cast<uint64_t>(h.second) << 32 | l.second);
+}
 template <typename T>
 __device__ __forceinline__ T swap_sum16(T a, T b) { return swap_sum<16>(a, b); }
 template <typename T>
@@ -226,6 +235,13 @@ __device__ __forceinline__ T xchg(T v, int lane) {
     else if constexpr (O == 8) r = dpp<0x140>(b);
     else r = static_cast<int>(swap_partner<O>(static_cast<unsigned>(b), lane));
     return __builtin_bit_cast(T, r);
+}
+
+template <int O>
+__device__ __forceinline__ double xchg(double v, int lane) {
+    const uint64_t x = __builtin_bit_cast(uint64_t, v);
+    const unsigned l = xchg<O>(static_cast<unsigned>(x), lane), h = xchg<O>(static_cast<unsigned>(x >> 32), lane);
+    return __builtin_bit_cast(double, static_cast<uint64_t>(h) << 32 | l);
 }
 
 // Sums NV per-lane values (NV a power of two <= 64) over the wave with NV - 1

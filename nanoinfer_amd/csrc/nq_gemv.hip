@@ -2577,10 +2577,11 @@ nq_status linear_q8_impl(const void* x, nq_dtype x_dtype, const int8_t* q, const
     const bool general = !fast && !long_k;
     const TileCall tile{x_dtype == NQ_F32 ? TileX::F32 : TileX::F16, x, reinterpret_cast<const uint8_t*>(q), false, w_scale,
                         false, 0, nullptr, bias, y, y_dtype == NQ_F32 ? kTileF32 : kTileF16, m, n, k, !operands};
-    // Short K stays on the element kernel, a column per lane: k <= 256 up to 2 rows of x, k <= 112
-    // past them (us, element kernel / gemv_any: m = 1, n = 2358, k = 65 3.0 / 3.6; m = 2, n = 6462,
-    // k = 87 3.8 / 4.7; m = 5, n = 426, k = 51 3.8 / 5.7; m = 2, n = 5373, k = 281 4.3 / 4.5).
-    if (path == NQ_PATH_AUTO && general && m <= 8 && k > (m <= 2 ? 256 : 112) && tile_gemm_ok(false, m, n, k, 0)) return gemv_any(tile, s);
+    // Short K stays on the element kernel, a column per lane: k <= 256 for one row of x, 160 for
+    // two, 112 past them (us, element kernel / gemv_any: m = 1, n = 2358, k = 65 3.0 / 3.4; m = 2, k =
+    // 65 to 96 1.11 times, 193 to 256 0.97; m = 5, n = 426, k = 51 3.7 / 4.6; 5 to 8 rows, k = 113 to
+    // 128 0.84 times).
+    if (path == NQ_PATH_AUTO && general && m <= 8 && k > (m == 1 ? 256 : m == 2 ? 160 : 112) && tile_gemm_ok(false, m, n, k, 0)) return gemv_any(tile, s);
     if (path == NQ_PATH_AUTO && wq_tile_route(false, x_dtype == NQ_F32, false, general, !operands, m, n, k, 0, ws ? ws_bytes : 0))
         return tile_gemm(tile, ws, ws_bytes, s);
     NQ_REQUIRE(!mfma || operands, NQ_BAD_ARG,

@@ -13,8 +13,8 @@
 //
 // Bound by latency on small weights and by the activation re-reads (one per R weight
 // rows) at 8 rows. us, element kernel -> this: Q8 fp32 x, n = 1001, k = 1003 m = 7 15.4 ->
-// 6.1; n = 1536, k = 8955 m = 1 37 -> 6.7, m = 8 272 -> 14; n = k = 9001 m = 2 146 -> 26
-// (3.1 TB/s); Q4G m = 1, n = 17920, k = 1531 83 -> 9.2; one int4 group per row, m = 8, n =
+// 5.5; n = 1536, k = 8955 m = 1 37 -> 6.5, m = 8 272 -> 13; n = k = 9001 m = 2 146 -> 26
+// (3.1 TB/s); Q4G m = 1, n = 17920, k = 1531 83 -> 9.0; one int4 group per row, m = 8, n =
 // 1536, k = 8955 7029 -> 13; W8A8 m = 2, n = k = 9001 135 -> 17 (4.7 TB/s).
 #include <hip/hip_runtime.h>
 
@@ -141,8 +141,10 @@ __global__ __launch_bounds__(256) void gemv_any_kernel(AnyArgs a) {
             }
         }
     }
-    // Lane l ends with the wave's sum of value l / (64 / NV).
-    wave_reduce_stage_bperm<NV, 32>(acc, lane);
+    // Lane l ends with the wave's sum of value l / (64 / NV). Doubles without the LDS: m = 7, n =
+    // 1001, k = 1003 6.1 -> 5.5 us, m = 8, n = 1536, k = 8955 13.7 -> 13.1.
+    if constexpr (I8) wave_reduce_stage_bperm<NV, 32>(acc, lane);
+    else wave_reduce_stage<NV, 32>(acc, lane);
     Acc sum = acc[0];
     constexpr int G = 64 / NV;
     if (kw > 1) {

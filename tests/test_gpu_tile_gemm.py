@@ -299,7 +299,7 @@ def test_kept_on_mfma(dev, nq, xdt, m, n, k, fmt, group):
 
 @gpu
 @pytest.mark.parametrize("xdt", [F32, F16])
-@pytest.mark.parametrize("m,n,k", [(1, 2358, 65), (2, 6462, 87), (2, 60, 255), (5, 426, 51), (8, 90, 111)])
+@pytest.mark.parametrize("m,n,k", [(1, 2358, 65), (2, 6462, 87), (2, 60, 159), (1, 60, 255), (5, 426, 51), (8, 90, 111)])
 def test_kept_on_elements(dev, nq, xdt, m, n, k):
     from nanoinfer_amd import _lib
     t, _ = _make(nq, "q8", n, k, 0, F32, None)
